@@ -61,11 +61,13 @@ struct LaunchClass {
 struct Chain {
     int cls, kernel, k, launches, blocks, mode, tails, tail_blocks;
     int alt_launches, alt_blocks, alt_mode;
+    int survey_words;  // active bands (tws_active.hip); 0: every row each launch
     bool operator<(const Chain& o) const {
         return std::tie(cls, kernel, k, launches, blocks, mode, tails, tail_blocks, alt_launches,
-                        alt_blocks, alt_mode) <
+                        alt_blocks, alt_mode, survey_words) <
                std::tie(o.cls, o.kernel, o.k, o.launches, o.blocks, o.mode, o.tails,
-                        o.tail_blocks, o.alt_launches, o.alt_blocks, o.alt_mode);
+                        o.tail_blocks, o.alt_launches, o.alt_blocks, o.alt_mode,
+                        o.survey_words);
     }
 };
 using GraphKey = std::vector<Chain>;
@@ -80,6 +82,14 @@ constexpr int kHdrInts = 4;  // per class: grids, tiles, table offset, unused
 // for its fallback table.
 constexpr int kMaxTail = 6;
 constexpr int kAltKernel = TWS_KERNEL_TILE_128x64, kAltK = 4;
+// Tasks a planned launch can hold (tws_active.hip), 1 MiB per class; a run
+// with more static tasks than this steps every row each launch.
+constexpr int kListRoom = 1 << 16;
+// The masks of the grid at pool offset `off` start at off / kBandShare,
+// rounded up to 8 bytes.
+constexpr size_t kBandShare = 1024;
+// Full launches from which a run's active bands are surveyed.
+constexpr int kActiveLaunches = 3;
 constexpr int kHdrCount = TWS_BATCH_MAX_CLASSES * (2 + kMaxTail);
 inline int tail_hdr(int cls, int r) { return TWS_BATCH_MAX_CLASSES + cls * kMaxTail + (r - 1); }
 inline int alt_hdr(int cls) { return TWS_BATCH_MAX_CLASSES * (1 + kMaxTail) + cls; }
@@ -111,6 +121,11 @@ struct tws_batch {
     hipStream_t aux[TWS_BATCH_MAX_CLASSES - 1] = {};  // branch streams of the chains
     hipEvent_t fork = nullptr;
     hipEvent_t join[TWS_BATCH_MAX_CLASSES - 1] = {};
+    // active bands: the masks of all grids (slot by slot, at band_at) and, per
+    // class, the planned tasks of its streaming chain
+    uint64_t* bands_dev = nullptr;
+    int4* lists[TWS_BATCH_MAX_CLASSES] = {};
+    int* list_counts = nullptr;
     bool use_graphs = true;
     std::map<GraphKey, hipGraphExec_t> graphs;
     int64_t captures = 0, replays = 0;
@@ -156,14 +171,30 @@ static hipError_t issue_chains(tws_batch* b, const GraphKey& chains) {
         const Chain& ch = chains[c];
         hipStream_t st = c == 0 ? b->stream : b->aux[c - 1];
         const int* hdr = b->hdr_dev + kHdrInts * ch.cls;
-        for (int j = 0; j < ch.launches && e == hipSuccess; ++j)
+        ActiveRun active;
+        if (ch.survey_words > 0) {
+            active.grids = b->table_dev;
+            active.hdr = hdr;
+            active.k = ch.k;
+            active.slots = stream_slots(ch.k, device_cus());
+            active.max_tasks = std::min(ch.blocks * 4, kListRoom);
+            active.survey_words = ch.survey_words;
+            active.list = b->lists[ch.cls];
+            active.count = b->list_counts + ch.cls;
+        }
+        for (int j = 0; j < ch.launches && e == hipSuccess; ++j) {
+            if (ch.survey_words > 0 && j % active_interval(ch.k) == 0)
+                e = launch_active(active, 0, j, j / active_interval(ch.k), st);
+            if (e != hipSuccess) break;
             e = ch.kernel == TWS_KERNEL_STREAM_128
-                    ? launch_stream_batch(ch.k, ch.mode, b->table_dev, hdr, ch.blocks, j, st)
+                    ? launch_stream_batch(ch.k, ch.mode, b->table_dev, hdr, ch.blocks, j,
+                                          active.list, active.count, st)
                     : launch_tile_batch(ch.kernel, ch.k, ch.mode, b->table_dev, hdr, ch.blocks, j, st);
+        }
         for (int r = 1; r <= kMaxTail && e == hipSuccess; ++r)
             if ((ch.tails >> r) & 1)
                 e = launch_stream_batch(r, ch.mode, b->table_dev, b->hdr_dev + kHdrInts * tail_hdr(ch.cls, r),
-                                        ch.tail_blocks, 0, st);
+                                        ch.tail_blocks, 0, nullptr, nullptr, st);
         for (int j = 0; j < ch.alt_launches && e == hipSuccess; ++j)
             e = launch_tile_batch(kAltKernel, kAltK, ch.alt_mode, b->table_dev,
                                   b->hdr_dev + kHdrInts * alt_hdr(ch.cls), ch.alt_blocks, j, st);
@@ -255,6 +286,10 @@ int tws_batch_create(int32_t max_grids, int64_t pool_bytes, void* stream, tws_ba
     e = hipMalloc(&base, cap);
     if (e != hipSuccess) { tws_batch_destroy(b); return hip_fail(e, "tws_batch_create: pool"); }
     b->pool.reset(base, cap);
+    // a grid's masks take at most 1/1408 of its planes (16 rows of 64 columns)
+    e = hipMalloc(&b->bands_dev, cap / kBandShare + 64);
+    if (e == hipSuccess) e = hipMalloc(&b->list_counts, sizeof(int) * TWS_BATCH_MAX_CLASSES);
+    if (e != hipSuccess) { tws_batch_destroy(b); return hip_fail(e, "tws_batch_create: bands"); }
     e = hipMalloc(&b->table_dev, sizeof(GridDesc) * 2 * (size_t)max_grids);
     if (e == hipSuccess) e = hipMalloc(&b->hdr_dev, sizeof(int) * kHdrInts * kHdrCount);
     if (e == hipSuccess) e = hipMalloc(&b->status_dev, sizeof(unsigned) * (size_t)max_grids);
@@ -286,6 +321,10 @@ int tws_batch_destroy(tws_batch* b) {
     if (b->hdr_host) (void)hipHostFree(b->hdr_host);
     if (b->table_copied) (void)hipEventDestroy(b->table_copied);
     if (b->fork) (void)hipEventDestroy(b->fork);
+    if (b->bands_dev) (void)hipFree(b->bands_dev);
+    if (b->list_counts) (void)hipFree(b->list_counts);
+    for (int4* p : b->lists)
+        if (p) (void)hipFree(p);
     for (int c = 0; c < TWS_BATCH_MAX_CLASSES - 1; ++c) {
         if (b->join[c]) (void)hipEventDestroy(b->join[c]);
         if (b->aux[c]) (void)hipStreamDestroy(b->aux[c]);
@@ -322,6 +361,8 @@ int tws_batch_add(tws_batch* b, int32_t width, int32_t height, const tws_params*
     s.g.bind(reinterpret_cast<float*>(b->pool.base() + off), width, height);
     s.g.params = *params;
     s.g.status = b->status_dev + id;
+    if (active_mask_bytes(s.g.pitch, height) > 0)
+        s.g.bands = b->bands_dev + (off / kBandShare + 7) / 8;
     int rc = grid_clear(s.g, b->stream);
     if (rc == TWS_OK) {
         hipError_t e = hipMemsetAsync(s.g.status, 0, sizeof(unsigned), b->stream);
@@ -556,6 +597,8 @@ int tws_batch_run(tws_batch* b) {
         const bool stream = lc.kernel == TWS_KERNEL_STREAM_128;
         const int first = n;
         int tiles = 0, max_steps = 0, mode = kModePlain;
+        int words = 0;       // of the streaming chain's grids' masks
+        bool banded = true;  // all of them keep masks
         const int cap = stream ? chain_cap(b, c, lc.k) : 0;
         if (stream && cap <= 0) return fail(TWS_ERR_NOMEM, "tws_batch_run: host allocation failed");
         for (int i = 0; i < b->max_grids; ++i) {
@@ -576,6 +619,11 @@ int tws_batch_run(tws_batch* b) {
                 mode = std::max(mode, kernel_mode(g));
                 max_steps = std::max(max_steps, s.steps);
             }
+            if (stream) {
+                g.word_begin = words;
+                words += g.tiles_x * g.band_words;
+                banded = banded && g.bands;
+            }
             g.tile_begin = tiles;  // first tile, or first task of the streaming kernel
             g.steps = s.steps;
             tiles += g.tiles_x * g.tiles_y;
@@ -584,7 +632,15 @@ int tws_batch_run(tws_batch* b) {
         set_header(b, c, n - first, tiles, first);
         // block bounds rounded up so small changes of the tile (task) count
         // reuse a graph; spare blocks exit
-        const int blocks = stream ? ((tiles + 3) / 4 + 63) / 64 * 64 : (tiles + 511) / 512 * 512;
+        int blocks = stream ? ((tiles + 3) / 4 + 63) / 64 * 64 : (tiles + 511) / 512 * 512;
+        int survey_words = 0;
+        if (stream && banded && max_steps / lc.k >= kActiveLaunches && lc.k > 1) {
+            const int slots = stream_slots(lc.k, device_cus());
+            if (std::max(tiles, slots) <= kListRoom) {
+                survey_words = (words + 63) / 64 * 64;
+                blocks = std::max(blocks, ((slots + 3) / 4 + 63) / 64 * 64);
+            }
+        }
         // a streaming class's tails (one launch per remainder r) and its
         // fallback tile table
         int tails = 0, tail_blocks = 0;
@@ -604,7 +660,7 @@ int tws_batch_run(tws_batch* b) {
         if (max_steps == 0 && tails == 0 && alt_steps == 0) continue;
         chains.push_back(Chain{c, lc.kernel, lc.k, (max_steps + lc.k - 1) / lc.k, blocks, mode,
                                tails, tail_blocks, (alt_steps + kAltK - 1) / kAltK,
-                               (alt_tiles + 511) / 512 * 512, alt_mode});
+                               (alt_tiles + 511) / 512 * 512, alt_mode, survey_words});
     }
     if (n == 0 && !direct) return TWS_OK;
     if (n > 0) {
@@ -690,6 +746,10 @@ int tws_batch_set_launch_classes(tws_batch* b, int32_t n, const int64_t* max_cel
             return fail(TWS_ERR_INVALID, "tws_batch_set_launch_classes: class bounds must be "
                         "positive and ascending");
     }
+    // the classes' lists of planned tasks, made once
+    for (int c = 0; c < n; ++c)
+        if (!b->lists[c]) TWS_HIP(hipMalloc(&b->lists[c], sizeof(int4) * kListRoom),
+                                  "tws_batch_set_launch_classes: task list");
     // branch streams and events for the chains beyond the first, made once
     for (int c = 0; c + 1 < n; ++c) {
         if (!b->aux[c]) TWS_HIP(hipStreamCreateWithFlags(&b->aux[c], hipStreamNonBlocking),

@@ -29,6 +29,16 @@ void GridState::bind(float* base, int w, int h) {
     parity = 0;
 }
 
+// Whether dry cells stay dry under these constants (tws_active.hip): a head
+// difference of at least 2^-83 must not vanish from a cell's total, which
+// takes K (unless it is 0: no flux at all) and C at least 2^-20, and heights
+// up to 2^60 must not overflow it.
+static bool dry_params(const tws_params& p) {
+    const float lo = 0x1p-20f, hi = 0x1p20f;
+    const float K = p.water_acceleration, C = p.cell_area_inv_timescaled;
+    return (K == 0.0f || (K >= lo && K <= hi)) && C >= lo && C <= hi;
+}
+
 GridDesc GridState::desc() const {
     GridDesc g{};
     g.b = b;
@@ -48,6 +58,9 @@ GridDesc GridState::desc() const {
     g.status = status;
     g.parity0 = parity;
     g.tile_group = tile_group;
+    g.bands = bands;
+    g.band_words = (int32_t)active_band_words(H);
+    g.dry_ok = dry_params(params) ? 1 : 0;
     const bool dispatch = params.boundary == TWS_BOUNDARY_REFERENCE_DISPATCH;
     g.upd_w = dispatch ? W / 16 * 16 : W;
     g.upd_h = dispatch ? H / 16 * 16 : H;

@@ -34,6 +34,13 @@ struct GridState {
     // 16 measured best at 4096^2 (+1.6% at k = 4, +2.8% at k = 6)
     int tile_group = 16;
 
+    // active bands (tws_active.hip): the grid's masks, and, outside a batch,
+    // room for a planned launch's tasks
+    uint64_t* bands = nullptr;
+    int4* list = nullptr;
+    int* list_count = nullptr;
+    int list_room = 0;
+
     static size_t bytes_for(int W, int H) {
         return sizeof(float) * (size_t)kPlanes * (size_t)pitch_of(W) * (size_t)H;
     }

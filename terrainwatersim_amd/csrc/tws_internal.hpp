@@ -62,6 +62,13 @@ struct GridDesc {
     // Streaming kernel in a batch: output rows per segment (tiles_x strips by
     // tiles_y segments, tasks numbered from tile_begin).
     int32_t seg_rows;
+    // Active bands (tws_active.hip): masks of the streaming kernel's strips,
+    // band_words words each (null: none kept); in a batch the first of its
+    // words among all grids'.
+    uint64_t* bands;
+    int32_t band_words, word_begin;
+    // Dry cells stay dry under these constants (dry_params).
+    int32_t dry_ok;
     unsigned int* status;    // bit 0: non-finite value seen
 };
 
@@ -137,9 +144,16 @@ hipError_t launch_stream_copy(const void* src, void* dst, int64_t bytes, int sha
 
 // The streaming step kernel (tws_stream.hip): one wavefront per strip
 // segment of `seg_rows` output rows and stream_shape() output columns.
+// With `list` and *count >= 0, a launch's tasks are the first *count entries
+// {strip, first row, end row, grid} instead (tws_active.hip).
 struct StreamPlan {
     int strips = 0, segs = 0, seg_rows = 0, blocks = 0;
+    const int4* list = nullptr;
+    const int* count = nullptr;
+    int list_cols = 0;  // output columns of the list's strips, at most the launch's own
 };
+// Longest segment worth a single round of wavefronts (rows).
+constexpr int kStreamSegRows = 320;
 // Output columns per strip at k steps per launch; false if k is not built.
 bool stream_shape(int k, int* ox);
 // A grid's tasks in a batched launch of the streaming kernel: strips of
@@ -151,11 +165,44 @@ bool stream_batch_plan(int W, int H, int k, int cap, int* strips, int* segs, int
 // compute units: the cap whose tasks, dealt to the XCDs and run on their
 // resident work-group slots in order, finish soonest.  May throw bad_alloc.
 int stream_batch_cap(const int* shapes, int n, int k, int cus);
+// Wavefronts of the streaming kernel that `cus` compute units run at once.
+int stream_slots(int k, int cus);
+
+// Active bands of a run of streaming launches (tws_active.hip).  Bands of
+// kActiveBand rows by one strip; what is wet at a survey stays within
+// kActiveReach rows and columns until the next one.
+constexpr int kActiveBand = 16, kActiveReach = 32;
+inline int active_interval(int k) { return kActiveReach / k; }  // launches per survey
+// 64-bit words per strip of a mask of a grid's bands, and the bytes of a
+// grid's masks (0: too low a grid to be worth it).  Strips are at least 64
+// columns wide.
+int64_t active_band_words(int H);
+inline int64_t active_mask_bytes(int64_t pitch, int H) {
+    return H < kActiveBand ? 0 : 4 * 8 * (pitch / 64) * active_band_words(H);
+}
+struct ActiveRun {
+    const GridDesc* grid = nullptr;   // single grid and its static plan, or
+    StreamPlan plan;
+    const GridDesc* grids = nullptr;  // a batch's table and header {grids,
+    const int* hdr = nullptr;         // tasks, offset, 0} in device memory
+    int k = 0, slots = 0;
+    int max_tasks = 0;                // tasks a launch has room for
+    int survey_words = 0;            // words of all grids
+    int4* list = nullptr;
+    int* count = nullptr;
+};
+// Surveys the state before launch launch_idx (of set `parity`, single grid)
+// and plans the launches until the next survey.  `round` counts the run's
+// surveys from 0.
+hipError_t launch_active(const ActiveRun& a, int parity, int launch_idx, int round,
+                         hipStream_t s);
+
 // Batched launch launch_idx of the streaming kernel (closed walls; `mode`
 // kModePlain or kModeRain, the highest of the table's grids): hdr_dev =
 // {grids, tasks, offset}; `blocks` is at least the work groups the tasks need.
 hipError_t launch_stream_batch(int k, int mode, const GridDesc* grids_dev, const int* hdr_dev,
-                               int blocks, int launch_idx, hipStream_t s);
+                               int blocks, int launch_idx, const int4* list, const int* count,
+                               hipStream_t s);
 // Segments of a W x H grid on a device of `cus` compute units: as many as
 // fill its wavefront slots once.
 StreamPlan stream_plan(int W, int H, int k, int cus);

@@ -128,6 +128,29 @@ __device__ __forceinline__ bool brush_reaches(float cx, float cy, float R2, int 
     return dx * dx + dy * dy < (double)R2 * (1.0 + 1e-6);
 }
 
+// The rows [lo, hi] of the domain on which the brush can reach a cell of
+// columns [x_lo, x_hi] (false: none): every row for which brush_reaches
+// holds, and at most two more at either end, where the amount is +0 * I.
+__device__ __forceinline__ bool brush_span(const GridDesc& g, int x_lo, int x_hi, double& lo,
+                                           double& hi) {
+    const float cx = g.rain_cx, cy = g.rain_cy;
+    const double dx = cx < (float)x_lo ? (double)x_lo - cx : (cx > (float)x_hi ? (double)cx - x_hi : 0.0);
+    const double left = (double)g.rain_R2 * (1.0 + 1e-6) - dx * dx;
+    if (!(left > 0.0)) return false;
+    const double r = sqrt(left) + 1.0;
+    lo = fmin(fmax(floor((double)cy - r), 0.0), (double)g.H);
+    hi = fmax(fmin(ceil((double)cy + r), (double)g.H - 1.0), -1.0);
+    return lo <= hi;
+}
+// The same as wave-uniform integers (lo > hi: none).
+__device__ __forceinline__ void brush_rows(const GridDesc& g, int x_lo, int x_hi, int& lo,
+                                           int& hi) {
+    double a, b;
+    const bool some = brush_span(g, x_lo, x_hi, a, b);
+    lo = __builtin_amdgcn_readfirstlane(some ? (int)a : 1);
+    hi = __builtin_amdgcn_readfirstlane(some ? (int)b : 0);
+}
+
 // flowUpdate.comp:53-59 for one cell: new outgoing flux from the products
 // p_i = g_i * K of the four head differences g_i (own head minus the
 // neighbour's, +x, -x, +y, -y), clamped at zero and scaled so the cell cannot

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <new>
 #include <vector>
@@ -18,7 +19,7 @@ struct tws_sim {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     float* base = nullptr;       // the grid's planes
-    double* aux = nullptr;       // volume partials + status word
+    double* aux = nullptr;       // volume partials + status words + active bands
     int kernel = TWS_KERNEL_TILE_128x64;
     int k = 4;
     double time_acc = 0.0;       // PerformSimulationStep accumulator
@@ -39,6 +40,21 @@ bool stream_usable(const GridState& gs) {
     return gs.params.boundary == TWS_BOUNDARY_CLOSED && gs.pitch * gs.H < ((int64_t)1 << 29);
 }
 
+// The active-band run of a grid's full launches of k steps; false if it is not
+// to be used.
+static constexpr int kActiveLaunches = 3;
+static bool plan_active(const GridState& gs, int k, int cus, ActiveRun* a) {
+    if (!gs.bands || !gs.desc().dry_ok) return false;
+    a->plan = stream_plan(gs.W, gs.H, k, cus);
+    a->k = k;
+    a->slots = stream_slots(k, cus);
+    a->max_tasks = std::min(gs.list_room, std::max(a->plan.blocks * 4, a->slots));
+    a->survey_words = (int)(a->plan.strips * active_band_words(gs.H));
+    a->list = gs.list;
+    a->count = gs.list_count;
+    return a->plan.blocks > 0 && a->max_tasks >= a->plan.strips * a->plan.segs;
+}
+
 // Streaming launches (tws_stream.hip): full launches of k steps, then the
 // remainder as launches of the largest built step counts that fit it (each
 // launch runs exactly its template's number of levels).
@@ -47,6 +63,12 @@ static int step_stream(GridState& gs, int k, int32_t n, hipStream_t stream, hipE
     int nl = 0;
     const int cus = device_cus();
     if (cus <= 0) return fail(TWS_ERR_DEVICE, "step: cannot query the device");
+    // The full launches of a call work on the active bands only, surveyed anew
+    // every few launches; from kActiveLaunches full launches on that pays for
+    // the survey.
+    ActiveRun active;
+    const bool lists = k > 1 && n / k >= kActiveLaunches && plan_active(gs, k, cus, &active);
+    int since = kActiveReach, round = 0;  // steps since the last survey, surveys
     int left = n;
     while (left > 0) {
         int kk = k;
@@ -55,15 +77,28 @@ static int step_stream(GridState& gs, int k, int32_t n, hipStream_t stream, hipE
             for (int c : ladder)
                 if (c <= left) { kk = c; break; }
         }
-        const StreamPlan plan = stream_plan(gs.W, gs.H, kk, cus);
+        StreamPlan plan = stream_plan(gs.W, gs.H, kk, cus);
         if (plan.blocks <= 0) return fail(TWS_ERR_INVALID, "step: bad stream launch (k %d)", kk);
         GridDesc g = gs.desc();
         g.steps = kk;
+        active.grid = &g;
+        if (lists && kk == k && since + k > kActiveReach) {
+            TWS_HIP(launch_active(active, gs.parity, nl, round++, stream), "step: active bands");
+            since = 0;
+        }
+        // (the last, shorter launches too, as far as the survey reaches)
+        if (lists && since + kk <= kActiveReach) {
+            plan.list = active.list;
+            plan.count = active.count;
+            stream_shape(k, &plan.list_cols);
+            plan.blocks = std::max(plan.blocks, (active.max_tasks + 3) / 4);
+        }
         if (ev && nl < ev_pairs) TWS_HIP(hipEventRecord(ev[2 * nl], stream), "step: event");
         TWS_HIP(launch_stream_single(kk, g, plan, gs.parity, stream), "step: stream kernel");
         if (ev && nl < ev_pairs) TWS_HIP(hipEventRecord(ev[2 * nl + 1], stream), "step: event");
         gs.parity ^= 1;
         left -= kk;
+        since += kk;
         ++nl;
     }
     if (launches) *launches = nl;
@@ -148,11 +183,24 @@ int tws_create(int32_t width, int32_t height, const tws_params* params, void* st
     }
     e = hipMalloc(&s->base, GridState::bytes_for(width, height));
     if (e != hipSuccess) { tws_destroy(s); return hip_fail(e, "tws_create: hipMalloc state"); }
-    e = hipMalloc(&s->aux, sizeof(double) * kVolumeParts + 256);
+    // active bands: the masks and a list with room for the tasks of any static
+    // plan (one per 64 columns and 8 rows) and of any device's wavefront slots
+    const int64_t masks = active_mask_bytes(GridState::pitch_of(width), height);
+    const int64_t room = masks == 0 ? 0
+        : std::max<int64_t>(GridState::pitch_of(width) / 64 * (height / 8), 4096);
+    const size_t fixed = sizeof(double) * kVolumeParts + 256;
+    e = hipMalloc(&s->aux, fixed + (size_t)masks + sizeof(int4) * (size_t)room);
     if (e != hipSuccess) { tws_destroy(s); return hip_fail(e, "tws_create: hipMalloc aux"); }
     s->g.bind(s->base, width, height);
     s->g.params = *params;
     s->g.status = reinterpret_cast<unsigned*>(s->aux + kVolumeParts);
+    if (masks > 0) {
+        char* base = reinterpret_cast<char*>(s->aux) + fixed;
+        s->g.list = reinterpret_cast<int4*>(base);
+        s->g.list_room = (int)std::min<int64_t>(room, INT32_MAX);
+        s->g.bands = reinterpret_cast<uint64_t*>(base + sizeof(int4) * (size_t)room);
+        s->g.list_count = reinterpret_cast<int*>(s->g.status + 32);
+    }
     int rc = grid_clear(s->g, s->stream);
     if (rc == TWS_OK) {
         e = hipMemsetAsync(s->g.status, 0, 256, s->stream);

@@ -185,7 +185,8 @@ __device__ __forceinline__ void f_fix(const GridDesc& g, int y, int x0, bool inn
 template <int KH, int MODE, bool BATCH>
 __global__ void __launch_bounds__(kStreamWaves * kWave, StreamGeom<KH>::WAVES_PER_SIMD)
 k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict__ hdr,
-         int launch_idx, int strips1, int segs1, int seg_rows1, int parity1) {
+         int launch_idx, int strips1, int segs1, int seg_rows1, int parity1,
+         const int4* __restrict__ list, const int* __restrict__ count, int list_cols) {
     constexpr bool RAIN = MODE == kModeRain;
     using G = StreamGeom<KH>;
     constexpr int kRing = G::RING;
@@ -199,7 +200,8 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
     // re-read each other's halo columns) meet in one L2.  The runs cover the
     // work groups that hold tasks, so the spare ones of a batch launch (its
     // block count is rounded up) fall evenly on the XCDs.
-    const int ntasks = BATCH ? hdr[1] : strips1 * segs1;
+    const int listed = list ? *count : -1;  // -1: the static plan
+    const int ntasks = listed >= 0 ? listed : BATCH ? hdr[1] : strips1 * segs1;
     const int nb = min((int)gridDim.x, (ntasks + kStreamWaves - 1) / kStreamWaves);
     const int bid = blockIdx.x;
     const int xcd = bid & 7, idx = bid >> 3;
@@ -208,6 +210,15 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
     const int blk = xcd * q + (xcd < rmd ? xcd : rmd) + idx;
     const int task = blk * kStreamWaves + wave;
     if (task >= ntasks) return;  // whole wavefront: no barrier follows
+    // a planned task: {strip, first row, end row, grid}
+    int4 planned = make_int4(0, 0, 0, 0);
+    if (listed >= 0) {
+        const int4 e = list[task];
+        planned.x = __builtin_amdgcn_readfirstlane(e.x);
+        planned.y = __builtin_amdgcn_readfirstlane(e.y);
+        planned.z = __builtin_amdgcn_readfirstlane(e.z);
+        planned.w = __builtin_amdgcn_readfirstlane(e.w);
+    }
     GridDesc g;
     int strips, seg_rows, parity, local;
     if constexpr (!BATCH) {
@@ -218,7 +229,7 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
         local = task;
     } else {
         const GridDesc* table = grids + hdr[2];
-        int lo = 0, hi = hdr[0] - 1;
+        int lo = planned.w, hi = listed >= 0 ? lo : hdr[0] - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
             if (table[mid].tile_begin <= task) lo = mid; else hi = mid - 1;
@@ -245,11 +256,13 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
         }
         parity = 0;
     }
-    const int seg = local / strips, strip = local - seg * strips;
-    const int Y0 = seg * seg_rows;
-    const int Y1 = min(g.H, Y0 + seg_rows);
+    const int seg = local / strips;
+    const int strip = listed >= 0 ? planned.x : local - seg * strips;
+    const int Y0 = listed >= 0 ? planned.y : seg * seg_rows;
+    const int Y1 = listed >= 0 ? planned.z : min(g.H, Y0 + seg_rows);
     if (Y0 >= Y1) return;
-    const int ox = strip * G::OX - G::HALOX;
+    const int out_cols = listed >= 0 ? list_cols : G::OX;
+    const int ox = strip * out_cols - G::HALOX;
     const int x0 = ox + lane * kSCPL;
     const int lx = lane * kSCPL;
     // x0 is even and at most pitch - 2: both columns lie in the row's pitch
@@ -264,7 +277,7 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
     // stored columns of this lane (both, or only the first one when the grid
     // ends between them: the second store then lands in the row padding,
     // which nothing reads)
-    const bool col_ok = lx >= G::HALOX && lx < G::HALOX + G::OX && x0 < g.W;
+    const bool col_ok = lx >= G::HALOX && lx < G::HALOX + out_cols && x0 < g.W;
     const bool second_in = x0 + 1 < g.W;
     const uint32_t plane_bytes = (uint32_t)(g.pitch * g.H * 4);  // < 2^31 (stream_usable)
     const __amdgpu_buffer_rsrc_t rd = plane_rsrc(g.d[parity ^ 1], plane_bytes);
@@ -274,9 +287,8 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
     const __amdgpu_buffer_rsrc_t r3 = plane_rsrc(g.f[parity ^ 1][3], plane_bytes);
     bool bad = false;
 
-    // rows of the b ring that the rain reaches (bit r & (kRing - 1)), wave-uniform
-    unsigned rain_rows = 0;
-    const bool rain_on = RAIN && g.rain_on != 0;
+    int rain_lo = 1, rain_hi = 0;
+    if (RAIN && g.rain_on != 0) brush_rows(g, ox, ox + kSEXW - 1, rain_lo, rain_hi);
 
     // Accepts input row y: writes b (and the rain amount) into the ring and
     // returns d with the first level's rain added.
@@ -285,17 +297,9 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
         const int slot = y & (kRing - 1);
 #pragma unroll
         for (int c = 0; c < kSCPL; ++c) s_b[wave][slot][lx + c] = b[c];
-        bool wet_row = false;
-        if (rain_on) {
-            wet_row = __builtin_amdgcn_readfirstlane(
-                          brush_reaches(g.rain_cx, g.rain_cy, g.rain_R2, ox, ox + kSEXW - 1, y, y)
-                              ? 1 : 0) != 0 &&
-                      (unsigned)y < (unsigned)g.H;
-        }
-        rain_rows = (rain_rows & ~(1u << slot)) | ((wet_row ? 1u : 0u) << slot);
 #pragma unroll
         for (int c = 0; c < kSCPL; ++c) dn[c] = d[c];
-        if (wet_row) {
+        if (RAIN && y >= rain_lo && y <= rain_hi) {
 #pragma unroll
             for (int c = 0; c < kSCPL; ++c) {
                 const bool in = x0 + c >= 0 && x0 + c < g.W;
@@ -472,7 +476,7 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
             if (j < KH) {
                 // the next level's rain, then its head
                 const int ring = yd & (kRing - 1);
-                if (RAIN && ((rain_rows >> ring) & 1u)) {
+                if (RAIN && yd >= rain_lo && yd <= rain_hi) {
 #pragma unroll
                     for (int c = 0; c < kSCPL; ++c) {
                         const bool in = x0 + c >= 0 && x0 + c < g.W;
@@ -568,8 +572,10 @@ bool stream_shape(int k, int* ox) {
     return stream_geom(k, ox, &w);
 }
 
-// Longest segment worth a single round of wavefronts (rows).
-static constexpr int kStreamSegRows = 320;
+int stream_slots(int k, int cus) {
+    int ox = 0, per_simd = 0;
+    return stream_geom(k, &ox, &per_simd) ? cus * 4 * per_simd : 0;
+}
 
 StreamPlan stream_plan(int W, int H, int k, int cus) {
     StreamPlan p{};
@@ -608,7 +614,8 @@ static hipError_t launch_stream_m(int k, const GridDesc& g1, const GridDesc* gri
 #define TWS_STREAM_CASE(KK)                                                                   \
     case KK:                                                                                  \
         hipLaunchKernelGGL((k_stream<KK, MODE, BATCH>), grid, block, 0, s, g1, grids, hdr,    \
-                           launch_idx, p.strips, p.segs, p.seg_rows, parity);                 \
+                           launch_idx, p.strips, p.segs, p.seg_rows, parity, p.list, p.count,   \
+                           p.list_cols);                                                      \
         break;
     switch (k) {
         TWS_STREAM_CASE(1)
@@ -727,10 +734,14 @@ int stream_batch_cap(const int* shapes, int n, int k, int cus) {
 }
 
 hipError_t launch_stream_batch(int k, int mode, const GridDesc* grids_dev, const int* hdr_dev,
-                               int blocks, int launch_idx, hipStream_t s) {
+                               int blocks, int launch_idx, const int4* list, const int* count,
+                               hipStream_t s) {
     if (blocks <= 0) return hipErrorInvalidValue;
     StreamPlan p{};
     p.blocks = blocks;
+    p.list = list;
+    p.count = count;
+    (void)stream_shape(k, &p.list_cols);
     const GridDesc g1{};
     switch (mode) {
         case kModePlain:
