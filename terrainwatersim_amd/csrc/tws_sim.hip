@@ -18,8 +18,10 @@ struct tws_sim {
     GridState g;
     hipStream_t stream = nullptr;
     bool own_stream = false;
-    float* base = nullptr;       // the grid's planes
-    double* aux = nullptr;       // volume partials + status words + active bands
+    // one block: the grid's planes, the volume partials and status words, the
+    // active bands' task list and masks
+    float* base = nullptr;
+    double* aux = nullptr;
     int kernel = TWS_KERNEL_TILE_128x64;
     int k = 4;
     double time_acc = 0.0;       // PerformSimulationStep accumulator
@@ -181,24 +183,24 @@ int tws_create(int32_t width, int32_t height, const tws_params* params, void* st
         if (e != hipSuccess) { delete s; return hip_fail(e, "tws_create: hipStreamCreate"); }
         s->own_stream = true;
     }
-    e = hipMalloc(&s->base, GridState::bytes_for(width, height));
-    if (e != hipSuccess) { tws_destroy(s); return hip_fail(e, "tws_create: hipMalloc state"); }
     // active bands: the masks and a list with room for the tasks of any static
     // plan (one per 64 columns and 8 rows) and of any device's wavefront slots
     const int64_t masks = active_mask_bytes(GridState::pitch_of(width), height);
     const int64_t room = masks == 0 ? 0
         : std::max<int64_t>(GridState::pitch_of(width) / 64 * (height / 8), 4096);
-    const size_t fixed = sizeof(double) * kVolumeParts + 256;
-    e = hipMalloc(&s->aux, fixed + (size_t)masks + sizeof(int4) * (size_t)room);
-    if (e != hipSuccess) { tws_destroy(s); return hip_fail(e, "tws_create: hipMalloc aux"); }
+    const size_t planes = GridState::bytes_for(width, height);  // a multiple of 256
+    const size_t aux = sizeof(double) * kVolumeParts + 256;
+    e = hipMalloc(&s->base, planes + aux + sizeof(int4) * (size_t)room + (size_t)masks);
+    if (e != hipSuccess) { tws_destroy(s); return hip_fail(e, "tws_create: hipMalloc state"); }
+    char* const block = reinterpret_cast<char*>(s->base);
+    s->aux = reinterpret_cast<double*>(block + planes);
     s->g.bind(s->base, width, height);
     s->g.params = *params;
     s->g.status = reinterpret_cast<unsigned*>(s->aux + kVolumeParts);
     if (masks > 0) {
-        char* base = reinterpret_cast<char*>(s->aux) + fixed;
-        s->g.list = reinterpret_cast<int4*>(base);
+        s->g.list = reinterpret_cast<int4*>(block + planes + aux);
         s->g.list_room = (int)std::min<int64_t>(room, INT32_MAX);
-        s->g.bands = reinterpret_cast<uint64_t*>(base + sizeof(int4) * (size_t)room);
+        s->g.bands = reinterpret_cast<uint64_t*>(s->g.list + room);
         s->g.list_count = reinterpret_cast<int*>(s->g.status + 32);
     }
     int rc = grid_clear(s->g, s->stream);
@@ -218,7 +220,6 @@ int tws_destroy(tws_sim* s) {
     if (!s) return TWS_OK;
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     if (s->base) (void)hipFree(s->base);
-    if (s->aux) (void)hipFree(s->aux);
     if (s->own_stream && s->stream) (void)hipStreamDestroy(s->stream);
     delete s;
     return TWS_OK;

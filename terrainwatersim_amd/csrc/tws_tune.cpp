@@ -2,12 +2,10 @@
 // table and the measuring autotuner.
 //
 // choose_launch() maps a grid size to (kernel variant, steps per launch).
-// The built-in table comes from an MI355X sweep over sizes 128^2..16384^2:
-// 64 x 64 tiles (16 waves up to 512^2, 8 waves up to 2816^2: small grids
-// are bound by the latency of one tile's levels, so more and smaller tiles
-// finish sooner), 128 x 64 tiles beyond (two work groups per CU so one loads
-// while the other computes), 5 steps per launch up to 4096^2 and 4 above;
-// grids above 2176^2 in closed walls take the streaming kernel at k = 6.
+// Grids up to 2176^2, and larger ones on other edges than closed walls, take
+// the tile launch that a measured table of launch times by rounds of tiles
+// makes the fastest (tile_launch); grids above 2176^2 in closed walls the
+// streaming kernel at k = 6.
 // tws_autotune() times every candidate (the tile variants and the streaming
 // kernel, each at k = 2..6 and 8) on scratch grids of the requested shapes
 // advanced as one batch and returns the winner; only tws_tune_record() enters a launch into
@@ -37,34 +35,38 @@ static int size_class(int64_t cells) {
     return c;
 }
 
-// 512^2 < cells <= 832^2: a CU holding two work groups of a 16-wave tile
-// runs both at half speed, so the best launch follows the number of rounds
-// of tiles on 256 CUs.  Each band below keeps one round count for its launch
-// over the whole band (square grids).  Same-run sweep, 1e9 cell-updates/s with a rain disc
-// (without), against 64x64 at k = 4:
-//   576^2  64x48_16W k=4: 108 (109) vs 81 (83)      1 round
-//   640^2  64x48_16W k=6: 102 (126) vs 95 (98)      2 rounds
-//   704^2  64x64_16W k=8: 119 (142) vs 111 (113)    2 rounds
-//   768^2  64x48_16W k=5: 133 (148) vs 126 (128)    2 rounds
-//   832^2  64x48_16W k=4: 142 (149) vs 120 (123)    2 rounds
-// Above 832^2 64x64 at k = 4 leads again (896^2: 142 vs at most 138 with rain).
-static void band_launch(int64_t cells, int* kernel, int* k) {
-    if (cells <= 576 * 576) {
-        *kernel = TWS_KERNEL_TILE_64x48_16W;
-        *k = 4;
-    } else if (cells <= 640 * 640) {
-        *kernel = TWS_KERNEL_TILE_64x48_16W;
-        *k = 6;
-    } else if (cells <= 704 * 704) {
-        *kernel = TWS_KERNEL_TILE_64x64_16W;
-        *k = 8;
-    } else if (cells <= 768 * 768) {
-        *kernel = TWS_KERNEL_TILE_64x48_16W;
-        *k = 5;
-    } else {
-        *kernel = TWS_KERNEL_TILE_64x48_16W;
-        *k = 4;
-    }
+// What a tile launch takes, by rounds of tiles.  A launch lasts as long as the
+// compute units (256) need for their rounds of work groups: a CU that holds two
+// runs both at half speed, so the time is a function of tiles / 256, rounded
+// up, and hardly of anything else; within the first round it grows a little
+// with every tile.  MI355X, us per launch of k steps on square grids of
+// 128^2..2304^2 (0.5 m sheet, closed walls; a rain disc adds 1-3%): few tiles,
+// then 256, 512, ... 2048 tiles.
+struct TileCost {
+    int kernel, k;
+    float few, rounds[8];
+};
+static const TileCost kTileCosts[] = {
+    {TWS_KERNEL_TILE_64x48_16W, 4, 9.3f, {12.7f, 17.9f, 21.4f, 25.4f, 30.6f, 35.3f, 39.9f, 44.4f}},
+    {TWS_KERNEL_TILE_64x48_16W, 5, 10.2f, {12.8f, 19.2f, 24.0f, 27.5f, 33.1f, 38.5f, 43.8f, 48.9f}},
+    {TWS_KERNEL_TILE_64x48_16W, 6, 11.2f, {13.3f, 19.6f, 26.2f, 30.1f, 35.5f, 41.3f, 47.5f, 53.2f}},
+    {TWS_KERNEL_TILE_64x48_16W, 8, 12.6f, {14.1f, 20.7f, 29.0f, 35.7f, 42.0f, 48.2f, 54.3f, 61.4f}},
+    {TWS_KERNEL_TILE_64x64_16W, 4, 11.2f, {16.4f, 20.3f, 26.0f, 32.2f, 38.6f, 44.5f, 50.1f, 55.9f}},
+    {TWS_KERNEL_TILE_64x64_16W, 5, 12.5f, {16.9f, 22.9f, 28.3f, 34.9f, 42.2f, 49.0f, 56.1f, 62.5f}},
+    {TWS_KERNEL_TILE_64x64_16W, 6, 13.7f, {17.5f, 25.0f, 31.0f, 38.4f, 46.1f, 53.6f, 62.0f, 69.5f}},
+    {TWS_KERNEL_TILE_64x64_16W, 8, 15.9f, {18.4f, 27.8f, 36.6f, 43.8f, 52.9f, 61.5f, 71.2f, 80.6f}},
+    {TWS_KERNEL_TILE_64x64, 4, 13.0f, {18.7f, 22.0f, 27.0f, 32.8f, 40.5f, 46.2f, 51.0f, 56.0f}},
+    {TWS_KERNEL_TILE_64x64, 5, 14.5f, {19.0f, 24.8f, 29.8f, 36.3f, 42.9f, 51.1f, 57.2f, 63.5f}},
+    {TWS_KERNEL_TILE_64x64, 6, 16.1f, {19.7f, 27.0f, 32.3f, 38.2f, 45.1f, 51.8f, 60.8f, 67.7f}},
+    {TWS_KERNEL_TILE_128x64, 5, 22.8f, {26.4f, 38.6f, 53.5f, 69.2f, 81.5f, 94.0f, 107.0f, 120.0f}},
+    {TWS_KERNEL_TILE_128x64, 6, 25.8f, {28.9f, 43.0f, 59.6f, 75.4f, 91.6f, 107.0f, 123.0f, 139.0f}},
+};
+
+static float launch_us(const TileCost& c, int64_t tiles) {
+    const float r = (float)tiles / 256.0f;
+    if (r <= 1.0f) return c.few + (c.rounds[0] - c.few) * r;
+    if (r <= 8.0f) return c.rounds[(tiles + 255) / 256 - 1];
+    return c.rounds[7] + (r - 8.0f) * 0.5f * (c.rounds[7] - c.rounds[5]);
 }
 
 void choose_launch(int width, int height, int* kernel, int* k) {
@@ -95,25 +97,16 @@ void choose_launch(int width, int height, int* kernel, int* k) {
 
 void tile_launch(int width, int height, int* kernel, int* k) {
     const int64_t cells = (int64_t)width * height;
-    // MI355X sweep (cell-updates/s; 0.5 m sheet on fBm terrain, with and without
-    // a rain disc; stale halo rows skipped in the 64-wide tiles):
-    //   <= 384^2   latency-bound, few tiles: 64x48 tiles over 16 waves of 3
-    //              rows put the grid on more CUs; ms per 1000 steps with rain:
-    //              256^2 1.70 (64x48, k = 8; 128 tiles) vs 2.10 (64x64, k = 8);
-    //              128^2 1.65 vs 2.07; 384^2 2.12 (64x48, k = 6; 160 tiles) vs
-    //              2.23 (64x64, k = 8) vs 3.11 (64x48, k = 8: 288 tiles, more
-    //              than one per CU)
-    //   <= 512^2   latency-bound: 64x64 tiles spread the grid over more CUs, and
-    //              16 waves of 4 rows (instead of 8 of 8) halve each wave's
-    //              serial work per level: 512^2 1.16e11 (64x64 16 waves, k = 8)
-    //              vs 8.7e10 (8 waves, k = 6) vs 5.1e10 (128x64, k = 5);
-    //              64x48 tiles: 2.93 ms per 1000 steps at best vs 2.38
-    //   <= 832^2   bands by tile rounds (band_launch)
-    //   <= 2304^2  64x64 tiles, 8 waves, k = 4: 2048^2 2.98e11 with rain
-    //              (3.31e11 without) vs 2.67e11 (2.91e11) for 128x64, k = 5;
-    //              1024^2 1.88e11 with rain vs 1.72e11; 2304^2 zero edge, ms
-    //              per 100 steps without (with) rain: 1.61 (1.62) vs 1.91
-    //              (1.81) for 128x64, k = 5
+    // Up to 1536^2 cells the launch that takes least per step by kTileCosts.
+    // Against one launch per band of sizes, us per 96 steps: 640^2 with rain 292
+    // vs 381, 864^2 with rain 413 vs 557, 960^2 428 vs 516, 1024^2 with rain 487
+    // vs 520, 1152^2 with rain 568 vs 644, 1408^2 693 vs 768, 100 x 8000 450 vs
+    // 517; 256^2 and 512^2 keep theirs.  Past 6 rounds the candidates come
+    // within a few percent and memory has its say:
+    //   <= 2304^2  64x64 tiles, 8 waves, k = 4: 2048^2 zero edge, us per 96
+    //              steps, 1343 vs 1428 for 64x64 over 16 waves, k = 5, with a
+    //              lake in closed walls 1314 vs 1382; 1800^2 zero edge 1086 vs
+    //              1150 for 128x64, k = 5
     //   <= 2816^2  64x64, k = 5 (zero edge, ms per 100 steps without (with)
     //              rain): 2560^2 2.09 (2.10) vs 2.31 (2.15) for 128x64, k = 5
     //              and 2.14 (2.16) at k = 4; 2816^2 2.50 (2.53) vs 2.57 (2.53)
@@ -122,17 +115,19 @@ void tile_launch(int width, int height, int* kernel, int* k) {
     //              3.08e11 (3.42e11) for 64x64, k = 4
     //   larger     128x64, k = 4: the 16384^2 dam-break 4.30e11 vs 4.10e11 at
     //              k = 5 (on an all-wet 16384^2 sheet k = 5 leads by 4%).
-    if (cells <= 256 * 256) {
-        *kernel = TWS_KERNEL_TILE_64x48_16W;
-        *k = 8;
-    } else if (cells <= 384 * 384) {
-        *kernel = TWS_KERNEL_TILE_64x48_16W;
-        *k = 6;
-    } else if (cells <= 512 * 512) {
-        *kernel = TWS_KERNEL_TILE_64x64_16W;
-        *k = 8;
-    } else if (cells <= 832 * 832) {
-        band_launch(cells, kernel, k);
+    if (cells <= 1536 * 1536) {
+        float best = 0.0f;
+        for (const TileCost& c : kTileCosts) {
+            TileShape sh{};
+            if (!tile_shape(c.kernel, c.k, &sh)) continue;
+            const int64_t tiles = (int64_t)((width + sh.ox - 1) / sh.ox) * ((height + sh.oy - 1) / sh.oy);
+            const float us = launch_us(c, tiles) / (float)c.k;
+            if (best == 0.0f || us < best) {
+                best = us;
+                *kernel = c.kernel;
+                *k = c.k;
+            }
+        }
     } else if (cells <= 2304 * 2304) {
         *kernel = TWS_KERNEL_TILE_64x64;
         *k = 4;
