@@ -15,14 +15,8 @@
 //             one length, as many as the device runs at once.
 // The launches until the next survey step these segments and nothing else.
 //
-// Why the dry cells are exactly +0: an outgoing flux is max(0, 0 F + (h - hn)
-// K), scaled by 0 / total = +0 where total > 0, and where nothing flows in the
-// depth is max(0, 0 + (0 - 0) C) = +0.  That leaves fluxes whose total
-// underflows to 0 (flowUpdate.comp:58 does not scale them) or overflows (0 *
-// Inf).  Neither can happen between heights that are 0 or between kLo and kHi
-// in size, which differ by at least 2^-23 kLo or not at all, under constants
-// that pass dry_params; k_survey calls a band dry only if its own heights and
-// those around it are such.
+// k_survey calls a band dry only where that holds to the bit: see
+// regular_height (tws_kernel_util.hpp).
 
 #include <hip/hip_runtime.h>
 
@@ -49,8 +43,6 @@ constexpr int kReachBands = kActiveReach / kBand;
 constexpr int kFullRounds = 4;
 constexpr int kMinRows = 16;          // shortest segment worth a wavefront
 
-constexpr uint32_t kLo = (uint32_t)(127 - 60) << 23, kHi = (uint32_t)(127 + 60) << 23;
-
 // Words of a grid's masks: any | left | right | active, strips x words each.
 __device__ __forceinline__ uint64_t* mask_of(const GridDesc& g, int strips, int which) {
     return g.bands + (int64_t)which * strips * g.band_words;
@@ -65,11 +57,6 @@ __device__ __forceinline__ int find_grid(int n, int i, First first) {
         if (first(mid) <= i) lo = mid; else hi = mid - 1;
     }
     return lo;
-}
-
-__device__ __forceinline__ bool regular(float b) {
-    const uint32_t u = __float_as_uint(b) & 0x7fffffffu;
-    return u == 0 || u - kLo <= kHi - kLo;
 }
 
 }  // namespace
@@ -168,8 +155,8 @@ k_survey(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
                 for (int r = -1; r <= kBand; ++r) {
                     const int y = min(max(y0 + r, 0), H - 1);
                     const vf2 b = *reinterpret_cast<const gfloat2*>(gptr(g.b) + (int64_t)y * g.pitch + xb);
-                    good[0] = good[0] && regular(b.x);
-                    good[1] = good[1] && regular(b.y);
+                    good[0] = good[0] && regular_height(b.x);
+                    good[1] = good[1] && regular_height(b.y);
                 }
                 ok = ok && (xb >= W || good[0]) && (xb + 1 >= W || good[1]);
             }

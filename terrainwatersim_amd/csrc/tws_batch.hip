@@ -62,12 +62,13 @@ struct Chain {
     int cls, kernel, k, launches, blocks, mode, tails, tail_blocks;
     int alt_launches, alt_blocks, alt_mode;
     int survey_words;  // active bands (tws_active.hip); 0: every row each launch
+    int dry;           // whether a tile chain's launches look for dry tiles
     bool operator<(const Chain& o) const {
         return std::tie(cls, kernel, k, launches, blocks, mode, tails, tail_blocks, alt_launches,
-                        alt_blocks, alt_mode, survey_words) <
+                        alt_blocks, alt_mode, survey_words, dry) <
                std::tie(o.cls, o.kernel, o.k, o.launches, o.blocks, o.mode, o.tails,
                         o.tail_blocks, o.alt_launches, o.alt_blocks, o.alt_mode,
-                        o.survey_words);
+                        o.survey_words, o.dry);
     }
 };
 using GraphKey = std::vector<Chain>;
@@ -88,6 +89,9 @@ constexpr int kListRoom = 1 << 16;
 // The masks of the grid at pool offset `off` start at off / kBandShare,
 // rounded up to 8 bytes.
 constexpr size_t kBandShare = 1024;
+// Bytes of a class's dry maps (4 MiB each of the two); a run with more tiles
+// looks for none.
+constexpr int64_t kDryRoom = 1 << 22;
 // Full launches from which a run's active bands are surveyed.
 constexpr int kActiveLaunches = 3;
 constexpr int kHdrCount = TWS_BATCH_MAX_CLASSES * (2 + kMaxTail);
@@ -126,6 +130,8 @@ struct tws_batch {
     uint64_t* bands_dev = nullptr;
     int4* lists[TWS_BATCH_MAX_CLASSES] = {};
     int* list_counts = nullptr;
+    // per class, a pair of dry maps of its tile chain's launches
+    uint8_t* dry_dev[TWS_BATCH_MAX_CLASSES] = {};
     bool use_graphs = true;
     std::map<GraphKey, hipGraphExec_t> graphs;
     int64_t captures = 0, replays = 0;
@@ -189,7 +195,8 @@ static hipError_t issue_chains(tws_batch* b, const GraphKey& chains) {
             e = ch.kernel == TWS_KERNEL_STREAM_128
                     ? launch_stream_batch(ch.k, ch.mode, b->table_dev, hdr, ch.blocks, j,
                                           active.list, active.count, st)
-                    : launch_tile_batch(ch.kernel, ch.k, ch.mode, b->table_dev, hdr, ch.blocks, j, st);
+                    : launch_tile_batch(ch.kernel, ch.k, ch.mode, b->table_dev, hdr, ch.blocks, j,
+                                        ch.dry ? dry_maps(b->dry_dev[ch.cls], kDryRoom, j) : DryMaps{}, st);
         }
         for (int r = 1; r <= kMaxTail && e == hipSuccess; ++r)
             if ((ch.tails >> r) & 1)
@@ -197,7 +204,7 @@ static hipError_t issue_chains(tws_batch* b, const GraphKey& chains) {
                                         ch.tail_blocks, 0, nullptr, nullptr, st);
         for (int j = 0; j < ch.alt_launches && e == hipSuccess; ++j)
             e = launch_tile_batch(kAltKernel, kAltK, ch.alt_mode, b->table_dev,
-                                  b->hdr_dev + kHdrInts * alt_hdr(ch.cls), ch.alt_blocks, j, st);
+                                  b->hdr_dev + kHdrInts * alt_hdr(ch.cls), ch.alt_blocks, j, DryMaps{}, st);
     }
     for (int c = 1; c < n && e == hipSuccess; ++c) {
         e = hipEventRecord(b->join[c - 1], b->aux[c - 1]);
@@ -324,6 +331,8 @@ int tws_batch_destroy(tws_batch* b) {
     if (b->bands_dev) (void)hipFree(b->bands_dev);
     if (b->list_counts) (void)hipFree(b->list_counts);
     for (int4* p : b->lists)
+        if (p) (void)hipFree(p);
+    for (uint8_t* p : b->dry_dev)
         if (p) (void)hipFree(p);
     for (int c = 0; c < TWS_BATCH_MAX_CLASSES - 1; ++c) {
         if (b->join[c]) (void)hipEventDestroy(b->join[c]);
@@ -634,6 +643,8 @@ int tws_batch_run(tws_batch* b) {
         // reuse a graph; spare blocks exit
         int blocks = stream ? ((tiles + 3) / 4 + 63) / 64 * 64 : (tiles + 511) / 512 * 512;
         int survey_words = 0;
+        const int dry = !stream && max_steps > 2 * lc.k && tile_looks(lc.kernel, lc.k) && tiles >= kDryTiles &&
+                        (int64_t)tiles * kDryTileBytes <= kDryRoom;
         if (stream && banded && max_steps / lc.k >= kActiveLaunches && lc.k > 1) {
             const int slots = stream_slots(lc.k, device_cus());
             if (std::max(tiles, slots) <= kListRoom) {
@@ -660,7 +671,7 @@ int tws_batch_run(tws_batch* b) {
         if (max_steps == 0 && tails == 0 && alt_steps == 0) continue;
         chains.push_back(Chain{c, lc.kernel, lc.k, (max_steps + lc.k - 1) / lc.k, blocks, mode,
                                tails, tail_blocks, (alt_steps + kAltK - 1) / kAltK,
-                               (alt_tiles + 511) / 512 * 512, alt_mode, survey_words});
+                               (alt_tiles + 511) / 512 * 512, alt_mode, survey_words, dry});
     }
     if (n == 0 && !direct) return TWS_OK;
     if (n > 0) {
@@ -750,6 +761,9 @@ int tws_batch_set_launch_classes(tws_batch* b, int32_t n, const int64_t* max_cel
     for (int c = 0; c < n; ++c)
         if (!b->lists[c]) TWS_HIP(hipMalloc(&b->lists[c], sizeof(int4) * kListRoom),
                                   "tws_batch_set_launch_classes: task list");
+    for (int c = 0; c < n; ++c)
+        if (!b->dry_dev[c]) TWS_HIP(hipMalloc(&b->dry_dev[c], 2 * (size_t)kDryRoom),
+                                    "tws_batch_set_launch_classes: dry maps");
     // branch streams and events for the chains beyond the first, made once
     for (int c = 0; c + 1 < n; ++c) {
         if (!b->aux[c]) TWS_HIP(hipStreamCreateWithFlags(&b->aux[c], hipStreamNonBlocking),

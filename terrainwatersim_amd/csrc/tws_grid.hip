@@ -29,14 +29,15 @@ void GridState::bind(float* base, int w, int h) {
     parity = 0;
 }
 
-// Whether dry cells stay dry under these constants (tws_active.hip): a head
-// difference of at least 2^-83 must not vanish from a cell's total, which
-// takes K (unless it is 0: no flux at all) and C at least 2^-20, and heights
-// up to 2^60 must not overflow it.
+// Whether dry cells stay dry under these constants (regular_height,
+// tws_kernel_util.hpp): a head difference of at least 2^-83 must not vanish
+// from a cell's total, which takes K (unless it is 0: no flux at all) and C at
+// least 2^-20, heights up to 2^60 must not overflow it, and nothing may flow
+// in from outside the grid.
 static bool dry_params(const tws_params& p) {
     const float lo = 0x1p-20f, hi = 0x1p20f;
     const float K = p.water_acceleration, C = p.cell_area_inv_timescaled;
-    return (K == 0.0f || (K >= lo && K <= hi)) && C >= lo && C <= hi;
+    return (p.boundary == TWS_BOUNDARY_CLOSED || p.ghost_alpha == 0.0f) && (K == 0.0f || (K >= lo && K <= hi)) && C >= lo && C <= hi;
 }
 
 GridDesc GridState::desc() const {

@@ -40,6 +40,10 @@ struct GridState {
     int4* list = nullptr;
     int* list_count = nullptr;
     int list_room = 0;
+    // a pair of dry maps of the tile kernels' launches (DryMaps), dry_bytes
+    // each; outside a batch, which keeps them per class
+    uint8_t* dry = nullptr;
+    int64_t dry_bytes = 0;
 
     static size_t bytes_for(int W, int H) {
         return sizeof(float) * (size_t)kPlanes * (size_t)pitch_of(W) * (size_t)H;

@@ -104,6 +104,20 @@ __device__ __forceinline__ bool nonfinite5(float a, float b, float c, float d, f
            !__builtin_isfinite(d) | !__builtin_isfinite(e);
 }
 
+// Dry cells stay dry: a cell with depth +0 and flux +0 keeps both through a
+// step unless a neighbour drains into it, to the bit.  Its outgoing fluxes are
+// max(0, 0 F + (h - hn) K), scaled by 0 / total = +0 where total > 0, and where
+// nothing flows in its depth is max(0, 0 + (0 - 0) C) = +0.  That leaves fluxes
+// whose total underflows to 0 (flowUpdate.comp:58 does not scale them) or
+// overflows (0 * Inf).  Neither can happen between heights that are 0 or
+// between 2^-60 and 2^60 in size, which differ by at least 2^-83 or not at
+// all, under the constants that set GridDesc::dry_ok.
+__device__ __forceinline__ bool regular_height(float b) {
+    constexpr uint32_t lo = (uint32_t)(127 - 60) << 23, hi = (uint32_t)(127 + 60) << 23;
+    const uint32_t u = __float_as_uint(b) & 0x7fffffffu;
+    return u == 0 || u - lo <= hi - lo;
+}
+
 // waterBrush.comp:26-28, one texel: saturate(1 - dot(c-p, c-p)/R^2) * I.
 __device__ __forceinline__ float brush_amount(float cx, float cy, float I, float R2, int x, int y) {
     const float tx = cx - (float)x;

@@ -21,6 +21,7 @@
 // the FP32 restatement regardless of tile shape or steps per launch.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "tws_internal.hpp"
 #include "tws.h"
@@ -40,7 +41,7 @@ struct TileGrid {
     unsigned int* status;
     int32_t pitch, W, H;
     int32_t tiles_x, tiles_y, tile_begin, tile_group;
-    int32_t steps, parity0, boundary, rain_on;
+    int32_t steps, parity0, boundary, rain_on, dry_ok;
     float F, K, C, ghost_alpha;
     float rain_cx, rain_cy, rain_I, rain_R2;
 
@@ -53,9 +54,25 @@ struct TileGrid {
 __host__ __device__ inline TileGrid tile_grid(const GridDesc& g) {
     return TileGrid{const_cast<float*>(g.b), g.status, (int32_t)g.pitch, g.W, g.H, g.tiles_x,
                     g.tiles_y, g.tile_begin, g.tile_group, g.steps, g.parity0, g.boundary,
-                    g.rain_on, g.F, g.K, g.C, g.ghost_d, g.rain_cx, g.rain_cy, g.rain_I,
+                    g.rain_on, g.dry_ok, g.F, g.K, g.C, g.ghost_d, g.rain_cx, g.rain_cy, g.rain_I,
                     g.rain_R2};
 }
+
+struct OneGrid {
+    static constexpr bool kTable = false, kLooks = false;
+    TileGrid g;
+};
+struct GridTable {
+    static constexpr bool kTable = true, kLooks = false;
+    const GridDesc* grids;
+    const int* hdr;
+    int launch_idx;
+};
+template <class Base>
+struct Looking : Base {
+    static constexpr bool kLooks = true;
+    DryMaps dry;
+};
 
 // Tile (tx, ty) of a grid's tile list position lt: groups of tile_group tile
 // columns, row by row within a group, so the tiles in flight at once form a
@@ -83,9 +100,15 @@ __device__ __forceinline__ void tile_coords(const TileGrid& g, int lt, int& tx, 
 // 128 VGPRs at 128x64: +2.6% at k = 4, +7% at k = 6); the rain kernel has
 // the rain but not the edge masking (6 instead of 23 scalar spills: +0.6% to
 // +1.8% on closed-wall grids with rain).
-template <int CPL, int RPW, int NW, int KH, int MODE>
+// DRY: a tile is passed over while both buffer sets hold zeros there and
+// nothing wet is within its halo, i.e. in the tiles around (DryMaps).  A kernel
+// of its own: the code alone makes a launch of one tile per compute unit 4%
+// longer (256^2), waiting for the marks one of a single round of work groups
+// 5% (1500 x 1000).
+template <int CPL, int RPW, int NW, int KH, int MODE, bool DRY>
 __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int levels,
-                                          int parity) {
+                                          int parity, const uint8_t* dry_in,
+                                          uint8_t* dry_out) {
     constexpr bool GEN = MODE != kModePlain;   // rain source compiled in
     constexpr bool EDGE = MODE == kModeGeneral;  // reference-edge masking compiled in
     using G = TileGeom<CPL, RPW, NW, KH>;
@@ -105,14 +128,6 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
     const int lx = lane * CPL;   // tile-local column of this lane's first cell
     const int ly = wave * RPW;   // tile-local row of this wave's first row
     const int x0 = ox + lx;
-    // a wave whose rows lie wholly outside the rain disc skips the brush
-    // (wave-uniform, decided before the state occupies the registers)
-    const bool rain =
-        GEN && g.rain_on != 0 &&
-        __builtin_amdgcn_readfirstlane(brush_reaches(g.rain_cx, g.rain_cy, g.rain_R2, ox,
-                                                     ox + EXW - 1, oy + ly, oy + ly + RPW - 1)
-                                           ? 1 : 0) != 0;
-
     float d[RPW][CPL], f0[RPW][CPL], f1[RPW][CPL], f2[RPW][CPL], f3[RPW][CPL];
     // ghost cells: closed walls, or the reference's out-of-image reads
     const bool closed = !EDGE || g.boundary == TWS_BOUNDARY_CLOSED;
@@ -120,6 +135,38 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
     const float ghost_d = closed ? 0.0f : g.ghost_alpha, ghost_fw = ghost_d;
     unsigned inside = 0;  // bit r*CPL+c: cell inside the domain
     bool bad = false;
+
+    // The marks of this tile and the tiles around it: lane i < 9 reads those of
+    // neighbour (i % 3 - 1, i / 3 - 1).
+    static_assert(NW == 8 || NW == 16, "a tile's marks are one or two 8-byte words");
+    constexpr int kWords = NW / 8;
+    constexpr uint64_t kOnes = 0x0101010101010101ull;
+    const int64_t marks_at = g.tile_begin + ty * g.tiles_x + tx;
+    bool before = false;  // this wavefront's output was dry in the launch before
+    if constexpr (DRY)
+        if (dry_in) {
+            const int nx = tx + lane % 3 - 1, ny = ty + lane / 3 - 1;
+            bool around = true;
+            if (lane < 9 && nx >= 0 && nx < g.tiles_x && ny >= 0 && ny < g.tiles_y)
+#pragma unroll
+                for (int i = 0; i < kWords; ++i) {
+                    const uint64_t m = reinterpret_cast<const uint64_t*>(
+                        dry_in)[(g.tile_begin + ny * g.tiles_x + nx) * (int64_t)kWords + i];
+                    around = around && (lane == 4 ? (m & 2 * kOnes) == 2 * kOnes
+                                                  : ((m | m >> 1) & kOnes) == kOnes);
+                    if (lane == 4 && i == wave / 8) before = (m >> (wave % 8 * 8) & 3) != 0;
+                }
+            before = __ballot(before) != 0;
+            // the rain on any wavefront's rows keeps the whole tile
+            if (__ballot(!around) == 0 &&
+                !(GEN && g.rain_on != 0 &&
+                  __builtin_amdgcn_readfirstlane(brush_reaches(g.rain_cx, g.rain_cy, g.rain_R2, ox,
+                                                               ox + EXW - 1, oy, oy + EXH - 1)
+                                                     ? 1 : 0) != 0)) {
+                if (lane == 0) dry_out[marks_at * NW + wave] = 2;
+                return false;  // every wavefront of the group alike
+            }
+        }
 
     // ---- load -------------------------------------------------------------
     {
@@ -158,6 +205,15 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
             }
         }
     }
+    // a wave whose rows lie wholly outside the rain disc skips the brush
+    // (wave-uniform; decided while the state is on its way: 256^2 rain at k = 8,
+    // us per 96 steps, 160.5 against 162.5 before the loads)
+    const bool rain =
+        GEN && g.rain_on != 0 &&
+        __builtin_amdgcn_readfirstlane(brush_reaches(g.rain_cx, g.rain_cy, g.rain_R2, ox,
+                                                     ox + EXW - 1, oy + ly, oy + ly + RPW - 1)
+                                           ? 1 : 0) != 0;
+
     const bool edge_tile = ox < 0 || oy < 0 || ox + EXW > W || oy + EXH > H;
     const bool need_mask = EDGE && g.boundary != TWS_BOUNDARY_CLOSED && edge_tile;
     // Closed walls carry no flux either way.  The wall ghost makes every
@@ -338,45 +394,86 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
                     }
             }
         }
+        if constexpr (DRY) {
+            unsigned held = 0;  // bits of the lane's output
+#pragma unroll
+            for (int r = 0; r < RPW; ++r) {
+                const int yl = ly + r;
+                if (!(col_ok && yl >= G::HALOY && yl < EXH - G::HALOY && oy + yl < H)) continue;
+#pragma unroll
+                for (int c = 0; c < CPL; ++c)
+                    if (full || x0 + c < W)
+                        held |= __float_as_uint(d[r][c]) | __float_as_uint(f0[r][c]) |
+                                __float_as_uint(f1[r][c]) | __float_as_uint(f2[r][c]) |
+                                __float_as_uint(f3[r][c]);
+            }
+            bool dry = g.dry_ok != 0 && __ballot(held != 0) == 0;
+            if (dry) {  // on ground where dry cells stay dry
+                bool ok = true;
+                for (int r = 0; r < RPW; ++r) {
+                    const int yl = ly + r;
+                    if (!(col_ok && yl >= G::HALOY && yl < EXH - G::HALOY && oy + yl < H)) continue;
+                    for (int c = 0; c < CPL; ++c)
+                        ok = ok && (x0 + c >= W || regular_height(s_b[yl * EXW + lx + c]));
+                }
+                dry = __ballot(!ok) == 0;
+            }
+            if (lane == 0) dry_out[marks_at * NW + wave] = dry ? (before ? 2 : 1) : 0;
+        }
     }
     return bad;
 }
 
 // ---------------------------------------------------------------------------
 // Fused, temporally blocked step.  Grid: one block per tile of the flattened
-// tile list.  Single grid: `grids` is null, g1 (by value) is the grid and
-// the tile count is gridDim.x.  Batch: hdr = {number of grids, number of
-// tiles, offset} and grids[offset..] (ordered by tile_begin) live in device
-// memory, so a captured launch stays valid while grids come and go; blocks past the tile
-// count exit at once.  MODE is the highest kernel_mode of the launch's grids
+// tile list; blocks past the tile count exit at once.  The arguments are of the
+// launch's kind, since a launch of one round of tiles notices their size (a 256^2
+// rain grid at k = 8, us per launch: 13.35 with 108 bytes, 13.50 with 124):
+//   OneGrid    the grid by value;
+//   GridTable  hdr = {number of grids, number of tiles, offset} and
+//              grids[offset..] (ordered by tile_begin) in device memory, so a
+//              captured launch stays valid while grids come and go;
+//   Looking    either, looking for dry tiles.  MODE is the highest kernel_mode of the launch's grids
 // (chosen on the host from the descriptors).
 // At least 4 waves per SIMD (at most 128 VGPRs): 2 work groups of 512 per CU.
-template <int CPL, int RPW, int NW, int KH, int MODE>
+template <int CPL, int RPW, int NW, int KH, int MODE, class Args>
 __global__ void __launch_bounds__(NW * kWave, 4)
-k_tile(TileGrid g1, const GridDesc* __restrict__ grids, const int* __restrict__ hdr,
-       int launch_idx) {
+k_tile(Args args) {
+    constexpr bool DRY = Args::kLooks;
     // XCD-aware order: the hardware deals blocks to the 8 XCDs round robin;
     // give each XCD a contiguous run of tiles so neighbouring tiles (whose
     // halos overlap) share one L2.
-    const int ngrids = grids ? hdr[0] : 0;
-    const int total_tiles = grids ? hdr[1] : g1.tiles_x * g1.tiles_y;
-    if (grids) grids += hdr[2];  // this launch's segment of the batch table
+    int total_tiles;
+    if constexpr (Args::kTable) total_tiles = args.hdr[1];
+    else total_tiles = args.g.tiles_x * args.g.tiles_y;
     const int bid = blockIdx.x;
     if (bid >= total_tiles) return;
     const int xcd = bid & 7, idx = bid >> 3;
     const int q = total_tiles >> 3, rmd = total_tiles & 7;
-    const int tile = xcd * q + (xcd < rmd ? xcd : rmd) + idx;
+    int tile = xcd * q + (xcd < rmd ? xcd : rmd) + idx;
+    if constexpr (DRY) {
+        // Runs of 32 tiles only, dealt round the XCDs: water gathers in some
+        // part of a grid, and an XCD with a whole eighth of the tiles would
+        // step it alone (2048^2 with a lake over 27% of the tiles: 48 us a
+        // launch with eighths).
+        constexpr int kRun = 32;
+        const int dealt = total_tiles / (8 * kRun) * (8 * kRun);
+        tile = bid < dealt ? (idx / kRun * 8 + xcd) * kRun + idx % kRun : bid;
+    }
 
     TileGrid g;
-    if (!grids) {
-        g = g1;
-    } else {
-        int lo = 0, hi = ngrids - 1;
+    int launch_idx = 0;
+    if constexpr (Args::kTable) {
+        const GridDesc* grids = args.grids + args.hdr[2];  // this launch's segment of the table
+        launch_idx = args.launch_idx;
+        int lo = 0, hi = args.hdr[0] - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
             if (grids[mid].tile_begin <= tile) lo = mid; else hi = mid - 1;
         }
         g = tile_grid(grids[lo]);
+    } else {
+        g = args.g;
     }
     const int levels = min(KH, g.steps - launch_idx * KH);
     if (levels <= 0) return;
@@ -389,7 +486,14 @@ k_tile(TileGrid g1, const GridDesc* __restrict__ grids, const int* __restrict__ 
     if (parity) lt = g.tiles_x * g.tiles_y - 1 - lt;
     int tx, ty;
     tile_coords(g, lt, tx, ty);
-    const bool bad = tile_step<CPL, RPW, NW, KH, MODE>(g, tx, ty, levels, parity);
+    const uint8_t* dry_in = nullptr;
+    uint8_t* dry_out = nullptr;
+    if constexpr (DRY) {
+        dry_in = args.dry.in;
+        dry_out = args.dry.out;
+    }
+    const bool bad = tile_step<CPL, RPW, NW, KH, MODE, DRY>(g, tx, ty, levels, parity, dry_in,
+                                                            dry_out);
     if (__ballot(bad) != 0 && (threadIdx.x & (kWave - 1)) == 0) atomicOr(g.status, 1u);
 }
 
@@ -664,32 +768,55 @@ __global__ void __launch_bounds__(64) k_lane_shift_probe(int* out) {
 
 static dim3 cell_grid(const GridDesc& g) { return dim3((g.W + 15) / 16, (g.H + 15) / 16); }
 
-template <int CPL, int RPW, int NW, int MODE>
-static hipError_t launch_tile_kg(int k, const GridDesc* grids_dev, const int* hdr,
-                                 const TileGrid& g1, int blocks, int launch_idx, hipStream_t s) {
-    const dim3 grid(blocks), block(NW * kWave);
-    switch (k) {
-        case 1: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 1, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        case 2: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 2, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        case 3: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 3, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        case 4: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 4, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        case 5: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 5, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        case 6: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 6, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        case 8: hipLaunchKernelGGL((k_tile<CPL, RPW, NW, 8, MODE>), grid, block, 0, s, g1, grids_dev, hdr, launch_idx); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+// Launches that look for dry tiles are built for the pairs the tile table
+// gives grids of many tiles.
+static constexpr bool dry_built(int cpl, int nw, int k) {
+    return nw == 8 && (k == 4 || k == 5) && (cpl == 1 || cpl == 2);
+}
+bool tile_looks(int kernel, int k) {
+    return (kernel == TWS_KERNEL_TILE_64x64 && dry_built(1, 8, k)) ||
+           (kernel == TWS_KERNEL_TILE_128x64 && dry_built(2, 8, k));
 }
 
-template <int CPL, int RPW, int NW>
-static hipError_t launch_tile_k(int k, int mode, const GridDesc* grids_dev, const int* hdr,
-                                const GridDesc* single, int blocks, int launch_idx,
+template <int CPL, int RPW, int NW, int MODE, class Args>
+static hipError_t launch_tile_kg(int k, const Args& args, int blocks, const DryMaps& dry,
+                                 hipStream_t s) {
+    const dim3 grid(blocks), block(NW * kWave);
+    auto launch = [&](auto steps) {
+        constexpr int KH = decltype(steps)::value;
+        if constexpr (dry_built(CPL, NW, KH)) {
+            if (dry.out) {
+                Looking<Args> look;
+                static_cast<Args&>(look) = args;
+                look.dry = dry;
+                hipLaunchKernelGGL((k_tile<CPL, RPW, NW, KH, MODE, Looking<Args>>), grid, block, 0,
+                                   s, look);
+                return hipGetLastError();
+            }
+        }
+        if (dry.out) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_tile<CPL, RPW, NW, KH, MODE, Args>), grid, block, 0, s, args);
+        return hipGetLastError();
+    };
+    switch (k) {
+        case 1: return launch(std::integral_constant<int, 1>{});
+        case 2: return launch(std::integral_constant<int, 2>{});
+        case 3: return launch(std::integral_constant<int, 3>{});
+        case 4: return launch(std::integral_constant<int, 4>{});
+        case 5: return launch(std::integral_constant<int, 5>{});
+        case 6: return launch(std::integral_constant<int, 6>{});
+        case 8: return launch(std::integral_constant<int, 8>{});
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <int CPL, int RPW, int NW, class Args>
+static hipError_t launch_tile_k(int k, int mode, const Args& args, int blocks, const DryMaps& dry,
                                 hipStream_t s) {
-    const TileGrid g1 = single ? tile_grid(*single) : TileGrid{};
     switch (mode) {
-        case kModePlain: return launch_tile_kg<CPL, RPW, NW, kModePlain>(k, grids_dev, hdr, g1, blocks, launch_idx, s);
-        case kModeRain: return launch_tile_kg<CPL, RPW, NW, kModeRain>(k, grids_dev, hdr, g1, blocks, launch_idx, s);
-        default: return launch_tile_kg<CPL, RPW, NW, kModeGeneral>(k, grids_dev, hdr, g1, blocks, launch_idx, s);
+        case kModePlain: return launch_tile_kg<CPL, RPW, NW, kModePlain>(k, args, blocks, dry, s);
+        case kModeRain: return launch_tile_kg<CPL, RPW, NW, kModeRain>(k, args, blocks, dry, s);
+        default: return launch_tile_kg<CPL, RPW, NW, kModeGeneral>(k, args, blocks, dry, s);
     }
 }
 
@@ -721,17 +848,17 @@ bool tile_shape(int kernel, int k, TileShape* out) {
     }
 }
 
-static hipError_t launch_tile_any(int kernel, int k, int mode, const GridDesc* grids_dev,
-                                  const int* hdr, const GridDesc* single, int blocks,
-                                  int launch_idx, hipStream_t s) {
+template <class Args>
+static hipError_t launch_tile_any(int kernel, int k, int mode, const Args& args, int blocks,
+                                  const DryMaps& dry, hipStream_t s) {
     if (blocks <= 0) return hipSuccess;
     switch (kernel) {
-        case TWS_KERNEL_TILE_128x128: return launch_tile_k<2, 8, 16>(k, mode, grids_dev, hdr, single, blocks, launch_idx, s);
-        case TWS_KERNEL_TILE_128x64: return launch_tile_k<2, 8, 8>(k, mode, grids_dev, hdr, single, blocks, launch_idx, s);
-        case TWS_KERNEL_TILE_256x64: return launch_tile_k<4, 4, 16>(k, mode, grids_dev, hdr, single, blocks, launch_idx, s);
-        case TWS_KERNEL_TILE_64x64: return launch_tile_k<1, 8, 8>(k, mode, grids_dev, hdr, single, blocks, launch_idx, s);
-        case TWS_KERNEL_TILE_64x64_16W: return launch_tile_k<1, 4, 16>(k, mode, grids_dev, hdr, single, blocks, launch_idx, s);
-        case TWS_KERNEL_TILE_64x48_16W: return launch_tile_k<1, 3, 16>(k, mode, grids_dev, hdr, single, blocks, launch_idx, s);
+        case TWS_KERNEL_TILE_128x128: return launch_tile_k<2, 8, 16>(k, mode, args, blocks, dry, s);
+        case TWS_KERNEL_TILE_128x64: return launch_tile_k<2, 8, 8>(k, mode, args, blocks, dry, s);
+        case TWS_KERNEL_TILE_256x64: return launch_tile_k<4, 4, 16>(k, mode, args, blocks, dry, s);
+        case TWS_KERNEL_TILE_64x64: return launch_tile_k<1, 8, 8>(k, mode, args, blocks, dry, s);
+        case TWS_KERNEL_TILE_64x64_16W: return launch_tile_k<1, 4, 16>(k, mode, args, blocks, dry, s);
+        case TWS_KERNEL_TILE_64x48_16W: return launch_tile_k<1, 3, 16>(k, mode, args, blocks, dry, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -742,14 +869,15 @@ int kernel_mode(const GridDesc& g) {
 }
 
 hipError_t launch_tile_batch(int kernel, int k, int mode, const GridDesc* grids_dev,
-                             const int* hdr_dev, int blocks, int launch_idx, hipStream_t s) {
-    return launch_tile_any(kernel, k, mode, grids_dev, hdr_dev, nullptr, blocks, launch_idx, s);
+                             const int* hdr_dev, int blocks, int launch_idx, const DryMaps& dry,
+                             hipStream_t s) {
+    return launch_tile_any(kernel, k, mode, GridTable{grids_dev, hdr_dev, launch_idx}, blocks, dry, s);
 }
 
-hipError_t launch_tile_single(int kernel, int k, const GridDesc& g, int launch_idx,
+hipError_t launch_tile_single(int kernel, int k, const GridDesc& g, const DryMaps& dry,
                               hipStream_t s) {
-    return launch_tile_any(kernel, k, kernel_mode(g), nullptr, nullptr, &g,
-                           g.tiles_x * g.tiles_y, launch_idx, s);
+    return launch_tile_any(kernel, k, kernel_mode(g), OneGrid{tile_grid(g)},
+                           g.tiles_x * g.tiles_y, dry, s);
 }
 
 hipError_t launch_twopass(const GridDesc* /*g_dev*/, const GridDesc& g, int parity,

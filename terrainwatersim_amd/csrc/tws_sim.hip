@@ -19,7 +19,7 @@ struct tws_sim {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     // one block: the grid's planes, the volume partials and status words, the
-    // active bands' task list and masks
+    // active bands' task list and masks, the tile kernels' dry maps
     float* base = nullptr;
     double* aux = nullptr;
     int kernel = TWS_KERNEL_TILE_128x64;
@@ -137,6 +137,7 @@ int step_grid(GridState& gs, int kernel, int k, int32_t n, hipStream_t stream, h
         if (launches) *launches = nl;
         return TWS_OK;
     }
+    const int full = n / k;
     int left = n;
     while (left > 0) {
         int kk = k;
@@ -151,8 +152,13 @@ int step_grid(GridState& gs, int kernel, int k, int32_t n, hipStream_t stream, h
             return fail(TWS_ERR_INVALID, "step: bad launch config %d/%d", kernel, kk);
         g.tile_begin = 0;
         g.steps = levels;
+        const int64_t tiles = (int64_t)g.tiles_x * g.tiles_y;
+        DryMaps dry;
+        if (kk == k && levels == k && full > 2 && tile_looks(kernel, k) && tiles >= kDryTiles &&
+            tiles * kDryTileBytes <= gs.dry_bytes)
+            dry = dry_maps(gs.dry, gs.dry_bytes, nl);
         TWS_HIP(rec(0), "step: event");
-        TWS_HIP(launch_tile_single(kernel, kk, g, 0, stream), "step: tile kernel");
+        TWS_HIP(launch_tile_single(kernel, kk, g, dry, stream), "step: tile kernel");
         TWS_HIP(rec(1), "step: event");
         gs.parity ^= 1;
         left -= levels;
@@ -188,15 +194,19 @@ int tws_create(int32_t width, int32_t height, const tws_params* params, void* st
     const int64_t masks = active_mask_bytes(GridState::pitch_of(width), height);
     const int64_t room = masks == 0 ? 0
         : std::max<int64_t>(GridState::pitch_of(width) / 64 * (height / 8), 4096);
+    // dry maps of the smallest tiles' output, 32 x 16 cells
+    s->g.dry_bytes = (int64_t)(width / 32 + 1) * (height / 16 + 1) * kDryTileBytes;
     const size_t planes = GridState::bytes_for(width, height);  // a multiple of 256
     const size_t aux = sizeof(double) * kVolumeParts + 256;
-    e = hipMalloc(&s->base, planes + aux + sizeof(int4) * (size_t)room + (size_t)masks);
+    const size_t lists = planes + aux + sizeof(int4) * (size_t)room + (size_t)masks;
+    e = hipMalloc(&s->base, lists + 2 * (size_t)s->g.dry_bytes);
     if (e != hipSuccess) { tws_destroy(s); return hip_fail(e, "tws_create: hipMalloc state"); }
     char* const block = reinterpret_cast<char*>(s->base);
     s->aux = reinterpret_cast<double*>(block + planes);
     s->g.bind(s->base, width, height);
     s->g.params = *params;
     s->g.status = reinterpret_cast<unsigned*>(s->aux + kVolumeParts);
+    s->g.dry = reinterpret_cast<uint8_t*>(block) + lists;
     if (masks > 0) {
         s->g.list = reinterpret_cast<int4*>(block + planes + aux);
         s->g.list_room = (int)std::min<int64_t>(room, INT32_MAX);
