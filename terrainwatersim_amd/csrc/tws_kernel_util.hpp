@@ -12,22 +12,27 @@ namespace tws {
 // ---------------------------------------------------------------------------
 // Cross-lane moves.  DPP wave_shr:1 (lane i reads lane i-1) and wave_shl:1
 // (lane i reads lane i+1).  The lane without a source (0 resp. 63, which sit
-// in the tile halo) reads 0, or `fill` in the *_or variants: heads are filled
-// with the lane's own head so the halo edge sees no gradient and does not
-// send every wave down the flux-scaling division.
+// in the tile's or strip's halo) reads 0, so the shift folds into the operation
+// that uses it.
 __device__ __forceinline__ float from_left_lane(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xF, 0xF, true));
 }
 __device__ __forceinline__ float from_right_lane(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float from_left_lane_or(float v, float fill) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(__float_as_int(fill), __float_as_int(v), 0x138, 0xF, 0xF, false));
+
+// Whether lane i is set in a wave-uniform mask, as a condition held in scalar
+// registers: no vector instruction.
+__device__ __forceinline__ bool lane_in(uint64_t mask) {
+    return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
-__device__ __forceinline__ float from_right_lane_or(float v, float fill) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(__float_as_int(fill), __float_as_int(v), 0x130, 0xF, 0xF, false));
+// Lanes, CPL columns each of a strip or tile `width` columns wide, whose flux of
+// level lev (from 0) can still reach an output column: those that hold any of
+// columns [2 lev + 1, width - 2 lev - 1).
+template <int CPL>
+__device__ __forceinline__ uint64_t live_lanes(int lev) {
+    const int edge = (2 * lev + 1) / CPL;  // lanes past use on either side
+    return (~0ull << edge) & (~0ull >> edge);
 }
 
 // Turns at the SIMD.  Wavefronts of different work groups that share a SIMD
@@ -168,9 +173,10 @@ __device__ __forceinline__ void brush_rows(const GridDesc& g, int x_lo, int x_hi
 // flowUpdate.comp:53-59 for one cell: new outgoing flux from the products
 // p_i = g_i * K of the four head differences g_i (own head minus the
 // neighbour's, +x, -x, +y, -y), clamped at zero and scaled so the cell cannot
-// drain below 0.
-__device__ __forceinline__ void flux_update_p(float F, float C, float d, float p0, float p1,
-                                              float p2, float p3, float& f0, float& f1,
+// drain below 0.  Lanes that are not `live` go unscaled: those whose flux reaches
+// no output any more, which then do not send their wave down the division.
+__device__ __forceinline__ void flux_update_p(float F, float C, float d, bool live, float p0,
+                                              float p1, float p2, float p3, float& f0, float& f1,
                                               float& f2, float& f3) {
     float o0 = fmaxf(0.0f, f0 * F + p0);
     float o1 = fmaxf(0.0f, f1 * F + p1);
@@ -178,7 +184,7 @@ __device__ __forceinline__ void flux_update_p(float F, float C, float d, float p
     float o3 = fmaxf(0.0f, f3 * F + p3);
     // flowUpdate.comp:57 summed pairwise, the order Mesa executes the reference in
     const float total = ((o0 + o1) + (o2 + o3)) * C;
-    if (total > d) {
+    if (total > d && live) {
         // flowUpdate.comp:58-59.  A dry cell on a slope (d = +0) gets s = +0;
         // an uploaded d = -0 gets s = -0 and signs the scaled fluxes, as the
         // division in the shader does.
@@ -192,7 +198,7 @@ __device__ __forceinline__ void flux_update_p(float F, float C, float d, float p
 __device__ __forceinline__ void flux_update(float F, float K, float C, float d, float g0,
                                             float g1, float g2, float g3, float& f0, float& f1,
                                             float& f2, float& f3) {
-    flux_update_p(F, C, d, g0 * K, g1 * K, g2 * K, g3 * K, f0, f1, f2, f3);
+    flux_update_p(F, C, d, true, g0 * K, g1 * K, g2 * K, g3 * K, f0, f1, f2, f3);
 }
 
 }  // namespace tws

@@ -446,11 +446,11 @@ k_stream(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict_
 #pragma unroll
                 for (int c = 0; c < kSCPL; ++c)
                     px[c] = (h0[c] - (c < kSCPL - 1 ? h0[c + 1] : h_right)) * K;
-                const float pl = from_left_lane_or(px[kSCPL - 1], 0.0f);
+                const float pl = from_left_lane(px[kSCPL - 1]);
 #pragma unroll
                 for (int c = 0; c < kSCPL; ++c) {
                     float o0 = fOwn[0][c], o1 = fOwn[1][c], o2 = fOwn[2][c], o3 = fOwn[3][c];
-                    flux_update_p(F, C, dOwn[c], px[c], -(c > 0 ? px[c - 1] : pl), py[c],
+                    flux_update_p(F, C, dOwn[c], true, px[c], -(c > 0 ? px[c - 1] : pl), py[c],
                                   pym[c], o0, o1, o2, o3);
                     FN[0][c] = o0; FN[1][c] = o1; FN[2][c] = o2; FN[3][c] = o3;
                 }
