@@ -72,10 +72,10 @@ struct GridDesc {
     int32_t dry_ok;
 };
 
-// Whether a grid must step on the two-pass kernels: the tile kernels update
-// every cell and rain on every cell, so they serve a reference-dispatch grid
-// only when its extents cover the whole grid.
-inline bool needs_twopass(const GridDesc& g) {
+// Whether the reference's dispatch shapes leave part of a grid as it is
+// (TWS_BOUNDARY_REFERENCE_DISPATCH with a side that is not a multiple of 16, or
+// of 32 where it rains).
+inline bool truncated(const GridDesc& g) {
     return g.upd_w < g.W || g.upd_h < g.H ||
            (g.rain_on != 0 && (g.brush_w < g.W || g.brush_h < g.H));
 }
@@ -100,9 +100,10 @@ struct TileShape {
 bool tile_shape(int kernel, int k, TileShape* out);
 
 // Step-kernel modes: what a launch compiles in.  Plain: closed walls without
-// rain.  Rain: closed walls, rain on some grids.  General: any edge mode.
-// Each mode runs every grid a lower mode can.
-constexpr int kModePlain = 0, kModeRain = 1, kModeGeneral = 2;
+// rain.  Rain: closed walls, rain on some grids.  General: any edge mode.  Each
+// of these runs every grid a lower one can.  Truncated: a grid whose last rows
+// or columns the reference's dispatch shapes leave out (not in a batch).
+constexpr int kModePlain = 0, kModeRain = 1, kModeGeneral = 2, kModeTruncated = 3;
 
 // Which tiles of a run of launches are dry: a byte per wavefront of a tile
 // (kDryTileBytes at most), 1 where its output rows came out dry, 2 where they

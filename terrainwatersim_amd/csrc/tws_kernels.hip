@@ -93,8 +93,8 @@ __device__ __forceinline__ void tile_coords(const TileGrid& g, int lt, int& tx, 
 
 // One tile: load its EXW x EXH block of state set `parity`, advance it
 // `levels` steps, store the valid interior into the other set.  Returns
-// whether this lane stored a non-finite value.  MODE (kModePlain,
-// kModeRain, kModeGeneral) compiles in only what the launch's grids use:
+// whether this lane stored a non-finite value.  MODE (kModePlain, kModeRain,
+// kModeGeneral, kModeTruncated) compiles in only what the launch's grids use:
 // the plain kernel has neither the rain source nor the reference-edge
 // masking (no per-cell domain masks, so no scalar spills and 111 instead of
 // 128 VGPRs at 128x64: +2.6% at k = 4, +7% at k = 6); the rain kernel has
@@ -110,7 +110,8 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
                                           int parity, const uint8_t* dry_in,
                                           uint8_t* dry_out) {
     constexpr bool GEN = MODE != kModePlain;   // rain source compiled in
-    constexpr bool EDGE = MODE == kModeGeneral;  // reference-edge masking compiled in
+    constexpr bool EDGE = MODE >= kModeGeneral;  // reference-edge masking compiled in
+    constexpr bool TAIL = MODE == kModeTruncated;  // cells no reference work group covers
     using G = TileGeom<CPL, RPW, NW, KH>;
     constexpr int EXW = G::EXW, EXH = G::EXH;
     __shared__ float s_b[EXH * EXW];
@@ -134,6 +135,10 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
     const float ghost_b = closed ? kWallHeight : 0.0f;
     const float ghost_d = closed ? 0.0f : g.ghost_alpha, ghost_fw = ghost_d;
     unsigned inside = 0;  // bit r*CPL+c: cell inside the domain
+    // The same for the cells the reference's truncating dispatch shapes leave as
+    // they are, and those its brush covers (GridDesc::upd_w, brush_w).
+    unsigned frozen = 0, brushed = 0;
+    const bool tail = TAIL && (ox + EXW > (W & ~15) || oy + EXH > (H & ~15));
     bool bad = false;
 
     // The marks of this tile and the tiles around it: lane i < 9 reads those of
@@ -196,6 +201,11 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
             for (int c = 0; c < CPL; ++c) {
                 const bool in = vin && (x0 + c < W);
                 inside |= (in ? 1u : 0u) << (r * CPL + c);
+                if constexpr (TAIL) {
+                    const int x = x0 + c;
+                    frozen |= (in && (x >= (W & ~15) || y >= (H & ~15)) ? 1u : 0u) << (r * CPL + c);
+                    brushed |= (in && x < (W & ~31) && y < (H & ~31) ? 1u : 0u) << (r * CPL + c);
+                }
                 s_b[(ly + r) * EXW + lx + c] = in ? vb[c] : ghost_b;
                 d[r][c] = in ? vd[c] : ghost_d;
                 f0[r][c] = in ? v0[c] : 0.0f;
@@ -262,7 +272,8 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
             for (int r = 0; r < RPW; ++r)
 #pragma unroll
                 for (int c = 0; c < CPL; ++c)
-                    if (inside & (1u << (r * CPL + c))) d[r][c] = d[r][c] + wet[r][c];
+                    if ((TAIL ? brushed : inside) & (1u << (r * CPL + c)))
+                        d[r][c] = d[r][c] + wet[r][c];
         }
 
         // ---- flux phase: flowUpdate.comp:34-62 ------------------------------
@@ -318,9 +329,14 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
                     px[c] = (h[r][c] - (c < CPL - 1 ? h[r][c + 1] : h_right)) * K;
                 const float px_left = from_left_lane(px[CPL - 1]);
 #pragma unroll
-                for (int c = 0; c < CPL; ++c)
+                for (int c = 0; c < CPL; ++c) {
+                    const float k0 = f0[r][c], k1 = f1[r][c], k2 = f2[r][c], k3 = f3[r][c];
                     flux_update_p(F, C, d[r][c], live, px[c], -(c > 0 ? px[c - 1] : px_left), py[c],
                                   -py_up[c], f0[r][c], f1[r][c], f2[r][c], f3[r][c]);
+                    if (TAIL && tail && (frozen & (1u << (r * CPL + c)))) {
+                        f0[r][c] = k0; f1[r][c] = k1; f2[r][c] = k2; f3[r][c] = k3;
+                    }
+                }
             }
 #pragma unroll
             for (int c = 0; c < CPL; ++c) py_up[c] = py[c];
@@ -362,7 +378,8 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
                 const float Y0z = r > 0 ? f2[r - 1][c] : f_up[c];
                 const float in = ((X1y + X0x) + Y1w) + Y0z;
                 const float out = ((f0[r][c] + f1[r][c]) + f2[r][c]) + f3[r][c];
-                d[r][c] = fmaxf(0.0f, d[r][c] + (in - out) * C);
+                const float nd = fmaxf(0.0f, d[r][c] + (in - out) * C);
+                if (!(TAIL && tail && (frozen & (1u << (r * CPL + c))))) d[r][c] = nd;
             }
         }
         if (need_mask) {
@@ -833,8 +850,11 @@ static hipError_t launch_tile_k(int k, int mode, const Args& args, int blocks, c
     switch (mode) {
         case kModePlain: return launch_tile_kg<CPL, RPW, NW, kModePlain>(k, args, blocks, dry, s);
         case kModeRain: return launch_tile_kg<CPL, RPW, NW, kModeRain>(k, args, blocks, dry, s);
-        default: return launch_tile_kg<CPL, RPW, NW, kModeGeneral>(k, args, blocks, dry, s);
+        case kModeGeneral: return launch_tile_kg<CPL, RPW, NW, kModeGeneral>(k, args, blocks, dry, s);
+        default: break;
     }
+    if constexpr (Args::kTable) return hipErrorInvalidValue;  // a batch takes no such grid
+    else return launch_tile_kg<CPL, RPW, NW, kModeTruncated>(k, args, blocks, dry, s);
 }
 
 template <int CPL, int RPW, int NW>
@@ -881,6 +901,7 @@ static hipError_t launch_tile_any(int kernel, int k, int mode, const Args& args,
 }
 
 int kernel_mode(const GridDesc& g) {
+    if (truncated(g)) return kModeTruncated;
     if (g.boundary != TWS_BOUNDARY_CLOSED) return kModeGeneral;
     return g.rain_on != 0 ? kModeRain : kModePlain;
 }

@@ -125,7 +125,7 @@ int step_grid(GridState& gs, int kernel, int k, int32_t n, hipStream_t stream, h
             return step_stream(gs, k, n, stream, ev, ev_pairs, launches);
         tile_launch(gs.W, gs.H, &kernel, &k);
     }
-    if (kernel == TWS_KERNEL_TWOPASS || needs_twopass(gs.desc())) {
+    if (kernel == TWS_KERNEL_TWOPASS) {
         for (int i = 0; i < n; ++i) {
             const GridDesc g = gs.desc();
             TWS_HIP(rec(0), "step: event");
