@@ -56,44 +56,109 @@ __device__ __forceinline__ float bilerp(float s00, float s01, float s10, float s
     return mip_lerp(mip_lerp(s00, s01, tx), mip_lerp(s10, s11, tx), ty);
 }
 
-constexpr int kMipBX = 64, kMipBY = 4;
+// Up to kMipLevels levels at once.  A work group owns a block of kMipSide >> 1
+// >> ... texels of each, and computes of every level what its texels of the next
+// one read too (one or two texels past its own where a side is odd), in LDS; the
+// last block of a row or column takes what the halving left over.  Bound by
+// launches and latency up to about 1024^2, by the one read of b and d above.
+constexpr int kMipLevels = 4;
+constexpr int kMipSide = 32;   // side of a block's first level
+constexpr int kMipReach = 40;  // what it computes of that level, at most: a last
+                               // block owns 32 + 7, an odd side needs 3 + 2 * 18
+constexpr int kMipRows = 8;    // wavefronts of a work group, a row of texels each
 
-// Level 1 from the state planes b (-> r) and d of set `parity` (-> a).
-__global__ void __launch_bounds__(kMipBX * kMipBY)
-k_mip_first(GridDesc g, int parity, float gb, float4* __restrict__ dst, int wd, int hd) {
-    const int i = blockIdx.x * kMipBX + (threadIdx.x & (kMipBX - 1));
-    const int j = blockIdx.y * kMipBY + (threadIdx.x / kMipBX);
-    if (i >= wd || j >= hd) return;
-    int x0, x1, y0, y1;
-    float tx, ty;
-    mip_axis(i, g.W, wd, x0, x1, tx);
-    mip_axis(j, g.H, hd, y0, y1, ty);
-    const int64_t r0 = (int64_t)y0 * g.pitch, r1 = (int64_t)y1 * g.pitch;
-    const float* b = g.b;
-    const float* d = g.d[parity];
-    const float r = bilerp(b[r0 + x0], b[r0 + x1], b[r1 + x0], b[r1 + x1], tx, ty);
-    const float a = bilerp(d[r0 + x0], d[r0 + x1], d[r1 + x0], d[r1 + x1], tx, ty);
-    const float c = bilerp(gb, gb, gb, gb, tx, ty);
-    dst[(int64_t)j * wd + i] = make_float4(r, c, c, a);
+struct MipSpan {
+    int first, own, end;  // computed: [first, end), written: [first, own)
+};
+
+// Texels of a level of `size`, `up` levels above the block's last one, whose
+// next level's span is `next`.
+__device__ __forceinline__ MipSpan mip_span(int block, bool last, int side, int up, int size,
+                                            int next_size, const MipSpan& next, bool have_next) {
+    MipSpan r;
+    r.first = min((block * side) << up, size);
+    r.own = last ? size : min(((block + 1) * side) << up, size);
+    r.end = r.own;
+    if (have_next && next.end > next.first) {
+        int i0, i1;
+        float t;
+        mip_axis(next.end - 1, size, next_size, i0, i1, t);
+        r.end = max(r.end, i1 + 1);
+    }
+    return r;
 }
 
-// Level l+1 from level l (both dense RGBA).
-__global__ void __launch_bounds__(kMipBX * kMipBY)
-k_mip_next(const float4* __restrict__ src, int ws, int hs, float4* __restrict__ dst, int wd,
-           int hd) {
-    const int i = blockIdx.x * kMipBX + (threadIdx.x & (kMipBX - 1));
-    const int j = blockIdx.y * kMipBY + (threadIdx.x / kMipBX);
-    if (i >= wd || j >= hd) return;
-    int x0, x1, y0, y1;
-    float tx, ty;
-    mip_axis(i, ws, wd, x0, x1, tx);
-    mip_axis(j, hs, hd, y0, y1, ty);
-    const float4 s00 = src[(int64_t)y0 * ws + x0], s01 = src[(int64_t)y0 * ws + x1];
-    const float4 s10 = src[(int64_t)y1 * ws + x0], s11 = src[(int64_t)y1 * ws + x1];
-    dst[(int64_t)j * wd + i] = make_float4(bilerp(s00.x, s01.x, s10.x, s11.x, tx, ty),
-                                           bilerp(s00.y, s01.y, s10.y, s11.y, tx, ty),
-                                           bilerp(s00.z, s01.z, s10.z, s11.z, tx, ty),
-                                           bilerp(s00.w, s01.w, s10.w, s11.w, tx, ty));
+// Levels 1..levels of a source of ws x hs: the planes b and d of set `parity`
+// (PLANES), or a level of the chain.  g = b = `gb` in every texel.
+template <bool PLANES>
+__global__ void __launch_bounds__(kWave * kMipRows)
+k_mip_block(GridDesc g, int parity, float gb, const float4* __restrict__ src, int ws, int hs,
+            float4* __restrict__ dst, int levels) {
+    __shared__ float2 s_mip[2][kMipReach * kMipReach];  // {r, a}
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int side = kMipSide >> (levels - 1);
+    const bool last_x = blockIdx.x + 1 == gridDim.x, last_y = blockIdx.y + 1 == gridDim.y;
+    MipSpan sx[kMipLevels], sy[kMipLevels];
+    int w[kMipLevels], h[kMipLevels];
+#pragma unroll
+    for (int l = 0; l < kMipLevels; ++l) {
+        w[l] = max(1, ws >> (l + 1));
+        h[l] = max(1, hs >> (l + 1));
+        sx[l] = sy[l] = MipSpan{0, 0, 0};
+    }
+#pragma unroll
+    for (int l = kMipLevels - 1; l >= 0; --l) {
+        if (l >= levels) continue;
+        constexpr int top = kMipLevels - 1;
+        const int n = l < top ? l + 1 : top;
+        const bool more = l + 1 < levels;
+        sx[l] = mip_span(blockIdx.x, last_x, side, levels - 1 - l, w[l], w[n], sx[n], more);
+        sy[l] = mip_span(blockIdx.y, last_y, side, levels - 1 - l, h[l], h[n], sy[n], more);
+    }
+    const float* d = parity ? g.d[1] : g.d[0];
+#pragma unroll
+    for (int l = 0; l < kMipLevels; ++l) {
+        if (l >= levels) break;
+        const int sw = l == 0 ? ws : w[l > 0 ? l - 1 : 0], sh = l == 0 ? hs : h[l > 0 ? l - 1 : 0];
+        const int i = sx[l].first + lane;
+        if (i < sx[l].end) {
+            int x0, x1;
+            float tx;
+            mip_axis(i, sw, w[l], x0, x1, tx);
+            for (int j = sy[l].first + wave; j < sy[l].end; j += kMipRows) {
+                int y0, y1;
+                float ty;
+                mip_axis(j, sh, h[l], y0, y1, ty);
+                float2 v;
+                if (l == 0 && PLANES) {
+                    const int64_t r0 = (int64_t)y0 * g.pitch, r1 = (int64_t)y1 * g.pitch;
+                    v.x = bilerp(g.b[r0 + x0], g.b[r0 + x1], g.b[r1 + x0], g.b[r1 + x1], tx, ty);
+                    v.y = bilerp(d[r0 + x0], d[r0 + x1], d[r1 + x0], d[r1 + x1], tx, ty);
+                } else if (l == 0) {
+                    const float4* r0 = src + (int64_t)y0 * ws;
+                    const float4* r1 = src + (int64_t)y1 * ws;
+                    const float4 s00 = r0[x0], s01 = r0[x1], s10 = r1[x0], s11 = r1[x1];
+                    v.x = bilerp(s00.x, s01.x, s10.x, s11.x, tx, ty);
+                    v.y = bilerp(s00.w, s01.w, s10.w, s11.w, tx, ty);
+                } else {
+                    const MipSpan &px = sx[l > 0 ? l - 1 : 0], &py = sy[l > 0 ? l - 1 : 0];
+                    const float2* up = s_mip[(l & 1) ^ 1];
+                    const float2* r0 = up + (y0 - py.first) * kMipReach - px.first;
+                    const float2* r1 = up + (y1 - py.first) * kMipReach - px.first;
+                    const float2 s00 = r0[x0], s01 = r0[x1], s10 = r1[x0], s11 = r1[x1];
+                    v.x = bilerp(s00.x, s01.x, s10.x, s11.x, tx, ty);
+                    v.y = bilerp(s00.y, s01.y, s10.y, s11.y, tx, ty);
+                }
+                s_mip[l & 1][(j - sy[l].first) * kMipReach + lane] = v;
+                if (i < sx[l].own && j < sy[l].own) {
+                    const float c = bilerp(gb, gb, gb, gb, tx, ty);
+                    dst[(int64_t)j * w[l] + i] = make_float4(v.x, c, c, v.y);
+                }
+            }
+        }
+        __syncthreads();
+        dst += (int64_t)w[l] * h[l];
+    }
 }
 
 // The small end of the chain in one work group: every level from one of at
@@ -129,8 +194,6 @@ k_mip_tail(const float4* src, int ws, int hs, float4* dst) {
     }
 }
 
-dim3 mip_grid(int wd, int hd) { return dim3((wd + kMipBX - 1) / kMipBX, (hd + kMipBY - 1) / kMipBY); }
-
 }  // namespace
 
 int mip_chain(int W, int H, int* levels, size_t* floats) {
@@ -160,28 +223,30 @@ int grid_mips(GridState& g, float gb_fill, float* dst, size_t capacity_floats, h
     float4* out = reinterpret_cast<float4*>(dst);
     const float4* prev = nullptr;
     int ws = g.W, hs = g.H;
-    for (int l = 1; l < levels; ++l) {
-        const int wd = g.W >> l > 0 ? g.W >> l : 1, hd = g.H >> l > 0 ? g.H >> l : 1;
-        if (l > 1 && (int64_t)wd * hd <= kTailTexels) {
-            // levels l .. levels-1 in one launch (their sizes follow the same
-            // halving rule, so the tail writes them where the loop would)
+    for (int left = levels - 1; left > 0;) {
+        if (prev && ws * (int64_t)hs <= kTailTexels) {
             hipLaunchKernelGGL(k_mip_tail, dim3(1), dim3(kTailThreads), 0, s, prev, ws, hs, out);
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return hip_fail(e, "mips: launch");
-            return TWS_OK;
+            left = 0;
+        } else {
+            const int n = left < kMipLevels ? left : kMipLevels, side = kMipSide >> (n - 1);
+            const int wl = ws >> n > 0 ? ws >> n : 1, hl = hs >> n > 0 ? hs >> n : 1;
+            const dim3 grid((wl + side - 1) / side, (hl + side - 1) / side);
+            if (prev)
+                hipLaunchKernelGGL((k_mip_block<false>), grid, dim3(kWave * kMipRows), 0, s, gd,
+                                   g.parity, gb_fill, prev, ws, hs, out, n);
+            else
+                hipLaunchKernelGGL((k_mip_block<true>), grid, dim3(kWave * kMipRows), 0, s, gd,
+                                   g.parity, gb_fill, prev, ws, hs, out, n);
+            for (int l = 0; l < n; ++l) {
+                prev = out;
+                ws = ws / 2 > 0 ? ws / 2 : 1;
+                hs = hs / 2 > 0 ? hs / 2 : 1;
+                out += (size_t)ws * hs;
+            }
+            left -= n;
         }
-        if (l == 1)
-            hipLaunchKernelGGL(k_mip_first, mip_grid(wd, hd), dim3(kMipBX * kMipBY), 0, s, gd,
-                               g.parity, gb_fill, out, wd, hd);
-        else
-            hipLaunchKernelGGL(k_mip_next, mip_grid(wd, hd), dim3(kMipBX * kMipBY), 0, s, prev,
-                               ws, hs, out, wd, hd);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_fail(e, "mips: launch");
-        prev = out;
-        out += (size_t)wd * hd;
-        ws = wd;
-        hs = hd;
     }
     return TWS_OK;
 }
