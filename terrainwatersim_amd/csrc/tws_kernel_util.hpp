@@ -70,6 +70,19 @@ typedef float vf4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) vf2 gfloat2;
 typedef __attribute__((address_space(1))) vf4 gfloat4;
 
+// A lane's element of a row: the row's address, made a scalar (it is the
+// same in every lane), plus the lane's byte offset zero-extended from 32
+// bits, so the load takes its base from scalar registers and needs no
+// per-lane 64-bit address.
+__device__ __forceinline__ const gfloat* at(const float* plane, int64_t row, uint32_t xbytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(plane + row);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    const char __attribute__((address_space(1)))* p =
+        (const char __attribute__((address_space(1)))*)(((uint64_t)hi << 32) | lo);
+    return (const gfloat*)(p + xbytes);
+}
+
 template <int N>
 __device__ __forceinline__ void vload(const gfloat* p, float (&o)[N]);
 template <>

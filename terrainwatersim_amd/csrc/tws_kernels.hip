@@ -174,57 +174,103 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
         }
 
     // ---- load -------------------------------------------------------------
+    // All loads of the wavefront are issued before the first is waited for, the
+    // terrain first: no branch surrounds them, from addresses clamped into the
+    // grid, and what lies outside it is replaced afterwards.  (A branch per row
+    // had every row wait for the one before, RPW round trips to memory.  MI355X,
+    // us before -> after: 1500 x 1000 sheet, 100 steps, 624 -> 588; 2048^2 with a
+    // lake, 100 steps, 1100 -> 1020; 256^2 rain, 1000 steps, 1596 -> 1562; 4096^2
+    // zero edge all wet, 96 steps, 4490 -> 4300.)
+    const bool edge_tile = ox < 0 || oy < 0 || ox + EXW > W || oy + EXH > H;
+    float vb[RPW][CPL];
     {
-        const gfloat* __restrict__ pb = gptr((const float*)g.base);
-        const gfloat* __restrict__ pd = gptr((const float*)g.d(parity));
-        const gfloat* __restrict__ p0 = gptr((const float*)g.f(parity, 0));
-        const gfloat* __restrict__ p1 = gptr((const float*)g.f(parity, 1));
-        const gfloat* __restrict__ p2 = gptr((const float*)g.f(parity, 2));
-        const gfloat* __restrict__ p3 = gptr((const float*)g.f(parity, 3));
+        // A row's address is wave-uniform.  Lanes of 16 cells, whose vector
+        // registers the loads fill, keep it in scalar ones; the others, whose
+        // residency many scalar registers cost, an offset from their first row's.
+        constexpr bool kRowScalar = CPL * RPW >= 16;
+        const int top = kRowScalar ? 0 : min(max(oy + ly, 0), H - 1);
+        const uint32_t xb = (uint32_t)min(max(x0, 0), g.pitch - CPL) * 4u;
+        auto load = [&](const float* plane, float (&v)[RPW][CPL]) {
 #pragma unroll
-        for (int r = 0; r < RPW; ++r) {
-            const int y = oy + ly + r;
-            const bool vin = (unsigned)y < (unsigned)H && x0 >= 0 && x0 < W;
-            float vb[CPL], vd[CPL], v0[CPL], v1[CPL], v2[CPL], v3[CPL];
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) vb[c] = vd[c] = v0[c] = v1[c] = v2[c] = v3[c] = 0.0f;
-            if (vin) {
-                const int64_t off = (int64_t)y * pitch + x0;
-                vload<CPL>(pb + off, vb);
-                vload<CPL>(pd + off, vd);
-                vload<CPL>(p0 + off, v0);
-                vload<CPL>(p1 + off, v1);
-                vload<CPL>(p2 + off, v2);
-                vload<CPL>(p3 + off, v3);
+            for (int r = 0; r < RPW; ++r) {
+                const int row = min(max(oy + ly + r, 0), H - 1) - top;
+                if constexpr (kRowScalar) vload<CPL>(at(plane, row * pitch, xb), v[r]);
+                else vload<CPL>(at(plane, top * pitch, xb + (uint32_t)row * (uint32_t)g.pitch * 4u), v[r]);
             }
+        };
+        load(g.base, vb);
+        load(g.d(parity), d);
+        load(g.f(parity, 0), f0);
+        load(g.f(parity, 1), f1);
+        load(g.f(parity, 2), f2);
+        load(g.f(parity, 3), f3);
+    }
+    // The brush amounts do not change from level to level: computed once, in
+    // registers across the loop (recomputing them per level measured 13%
+    // slower at 256^2, where waves under the disc are on the critical path),
+    // and only by waves under the disc.  Left to itself the compiler hoisted
+    // the divisions out of the loop into every wave.  While the loads are on
+    // their way, but for lanes of 16 cells, which have no registers to spare until
+    // the terrain is in LDS (3001 x 2777 zero edge, 60 steps: 1538 us against 1349).
+    // A wave whose rows lie wholly outside the disc skips the brush (wave-uniform).
+    float wet[RPW][CPL];
+    bool rain = false;
+    auto brush = [&]() {
+        rain = GEN && g.rain_on != 0 &&
+               __builtin_amdgcn_readfirstlane(brush_reaches(g.rain_cx, g.rain_cy, g.rain_R2, ox,
+                                                            ox + EXW - 1, oy + ly,
+                                                            oy + ly + RPW - 1)
+                                                  ? 1 : 0) != 0;
+        if (rain) {
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                const bool in = vin && (x0 + c < W);
-                inside |= (in ? 1u : 0u) << (r * CPL + c);
-                if constexpr (TAIL) {
-                    const int x = x0 + c;
-                    frozen |= (in && (x >= (W & ~15) || y >= (H & ~15)) ? 1u : 0u) << (r * CPL + c);
-                    brushed |= (in && x < (W & ~31) && y < (H & ~31) ? 1u : 0u) << (r * CPL + c);
-                }
-                s_b[(ly + r) * EXW + lx + c] = in ? vb[c] : ghost_b;
-                d[r][c] = in ? vd[c] : ghost_d;
-                f0[r][c] = in ? v0[c] : 0.0f;
-                f1[r][c] = in ? v1[c] : 0.0f;
-                f2[r][c] = in ? v2[c] : 0.0f;
-                f3[r][c] = in ? v3[c] : ghost_fw;
+            for (int r = 0; r < RPW; ++r)
+#pragma unroll
+                for (int c = 0; c < CPL; ++c)
+                    wet[r][c] = brush_amount(g.rain_cx, g.rain_cy, g.rain_I, g.rain_R2, x0 + c,
+                                             oy + ly + r);
+        } else {
+#pragma unroll
+            for (int r = 0; r < RPW; ++r)
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) wet[r][c] = 0.0f;
+        }
+    };
+    constexpr bool kBrushEarly = CPL * RPW < 16;
+    if constexpr (kBrushEarly) brush();
+    // The tile's cells outside the grid become ghosts.
+    auto in_grid = [&](int r, int c) {
+        return (unsigned)(oy + ly + r) < (unsigned)H && (unsigned)(x0 + c) < (unsigned)W;
+    };
+#pragma unroll
+    for (int r = 0; r < RPW; ++r)
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) {
+            const bool in = in_grid(r, c);
+            inside |= (in ? 1u : 0u) << (r * CPL + c);
+            if constexpr (TAIL) {
+                const int x = x0 + c, y = oy + ly + r;
+                frozen |= (in && (x >= (W & ~15) || y >= (H & ~15)) ? 1u : 0u) << (r * CPL + c);
+                brushed |= (in && x < (W & ~31) && y < (H & ~31) ? 1u : 0u) << (r * CPL + c);
             }
         }
+    if (edge_tile) {
+#pragma unroll
+        for (int r = 0; r < RPW; ++r)
+#pragma unroll
+            for (int c = 0; c < CPL; ++c) {
+                const bool in = in_grid(r, c);
+                vb[r][c] = in ? vb[r][c] : ghost_b;
+                d[r][c] = in ? d[r][c] : ghost_d;
+                f0[r][c] = in ? f0[r][c] : 0.0f;
+                f1[r][c] = in ? f1[r][c] : 0.0f;
+                f2[r][c] = in ? f2[r][c] : 0.0f;
+                f3[r][c] = in ? f3[r][c] : ghost_fw;
+            }
     }
-    // a wave whose rows lie wholly outside the rain disc skips the brush
-    // (wave-uniform; decided while the state is on its way: 256^2 rain at k = 8,
-    // us per 96 steps, 160.5 against 162.5 before the loads)
-    const bool rain =
-        GEN && g.rain_on != 0 &&
-        __builtin_amdgcn_readfirstlane(brush_reaches(g.rain_cx, g.rain_cy, g.rain_R2, ox,
-                                                     ox + EXW - 1, oy + ly, oy + ly + RPW - 1)
-                                           ? 1 : 0) != 0;
-
-    const bool edge_tile = ox < 0 || oy < 0 || ox + EXW > W || oy + EXH > H;
+#pragma unroll
+    for (int r = 0; r < RPW; ++r)
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) s_b[(ly + r) * EXW + lx + c] = vb[r][c];
     const bool need_mask = EDGE && g.boundary != TWS_BOUNDARY_CLOSED && edge_tile;
     // Closed walls carry no flux either way.  The wall ghost makes every
     // wall-ward flux the kernel computes max(0, f*F + (h - 1e30)*K) = +0 as
@@ -245,25 +291,7 @@ __device__ __forceinline__ bool tile_step(const TileGrid& g, int tx, int ty, int
             }
         }
     }
-    // The brush amounts do not change from level to level: computed once, in
-    // registers across the loop (recomputing them per level measured 13%
-    // slower at 256^2, where waves under the disc are on the critical path),
-    // and only by waves under the disc.  Left to itself the compiler hoisted
-    // the divisions out of the loop into every wave.
-    float wet[RPW][CPL];
-    if (rain) {
-#pragma unroll
-        for (int r = 0; r < RPW; ++r)
-#pragma unroll
-            for (int c = 0; c < CPL; ++c)
-                wet[r][c] = brush_amount(g.rain_cx, g.rain_cy, g.rain_I, g.rain_R2, x0 + c,
-                                         oy + ly + r);
-    } else {
-#pragma unroll
-        for (int r = 0; r < RPW; ++r)
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) wet[r][c] = 0.0f;
-    }
+    if constexpr (!kBrushEarly) brush();
     __syncthreads();  // s_b complete
 
     for (int lev = 0; lev < levels; ++lev) {
@@ -481,7 +509,7 @@ k_tile(Args args) {
     if constexpr (Args::kTable) total_tiles = args.hdr[1];
     else total_tiles = args.g.tiles_x * args.g.tiles_y;
     const int bid = blockIdx.x;
-    if (bid >= total_tiles) return;
+    if (Args::kTable && bid >= total_tiles) return;
     const int xcd = bid & 7, idx = bid >> 3;
     const int q = total_tiles >> 3, rmd = total_tiles & 7;
     int tile = xcd * q + (xcd < rmd ? xcd : rmd) + idx;
@@ -510,7 +538,7 @@ k_tile(Args args) {
         g = args.g;
     }
     const int levels = min(KH, g.steps - launch_idx * KH);
-    if (levels <= 0) return;
+    if (Args::kTable && levels <= 0) return;
     const int parity = (g.parity0 + launch_idx) & 1;
     // Every other launch walks the grid's tiles backwards, so it starts on the
     // tiles the launch before wrote last, whose state may still sit in the

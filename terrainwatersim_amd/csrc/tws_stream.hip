@@ -81,19 +81,6 @@ __device__ __forceinline__ int64_t row_base(const GridDesc& g, int y) {
     return (int64_t)min(max(y, 0), g.H - 1) * g.pitch;
 }
 
-// A lane's element of a row: the row's address, made a scalar (it is the
-// same in every lane), plus the lane's byte offset zero-extended from 32
-// bits, so the load takes its base from scalar registers and needs no
-// per-lane 64-bit address.
-__device__ __forceinline__ const gfloat* at(const float* plane, int64_t row, uint32_t xbytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(plane + row);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-    const char __attribute__((address_space(1)))* p =
-        (const char __attribute__((address_space(1)))*)(((uint64_t)hi << 32) | lo);
-    return (const gfloat*)(p + xbytes);
-}
-
 __device__ __forceinline__ void load_bd(const GridDesc& g, int parity, int y, uint32_t xb,
                                         float (&b)[kSCPL], float (&d)[kSCPL]) {
     const int64_t r = row_base(g, y);

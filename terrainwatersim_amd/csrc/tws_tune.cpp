@@ -107,12 +107,11 @@ void tile_launch(int width, int height, int* kernel, int* k) {
     //              steps, 1343 vs 1428 for 64x64 over 16 waves, k = 5, with a
     //              lake in closed walls 1314 vs 1382; 1800^2 zero edge 1086 vs
     //              1150 for 128x64, k = 5
-    //   <= 2816^2  64x64, k = 5 (zero edge, ms per 100 steps without (with)
-    //              rain): 2560^2 2.09 (2.10) vs 2.31 (2.15) for 128x64, k = 5
-    //              and 2.14 (2.16) at k = 4; 2816^2 2.50 (2.53) vs 2.57 (2.53)
-    //   <= 4096^2  128x64, k = 5: 3072^2 2.93 (2.90) ms vs 2.98 (3.01) for 64x64,
-    //              k = 5; 4096^2 3.36e11 with rain (3.59e11 without) vs
-    //              3.08e11 (3.42e11) for 64x64, k = 4
+    //   <= 3072^2  64x64, k = 5 (zero edge, all wet, us per 96 steps): 2500^2
+    //              1718 vs 1950 for 128x64, k = 5 and 1780 at k = 4; 3001 x 2777
+    //              2387 either way, and its smaller tiles pass over more once
+    //              the ground dries
+    //   <= 4096^2  128x64, k = 5: 4096^2 4300 us vs 4527 for 64x64, k = 5
     //   larger     128x64, k = 4: the 16384^2 dam-break 4.30e11 vs 4.10e11 at
     //              k = 5 (on an all-wet 16384^2 sheet k = 5 leads by 4%).
     if (cells <= 1536 * 1536) {
@@ -131,7 +130,7 @@ void tile_launch(int width, int height, int* kernel, int* k) {
     } else if (cells <= 2304 * 2304) {
         *kernel = TWS_KERNEL_TILE_64x64;
         *k = 4;
-    } else if (cells <= 2816 * 2816) {
+    } else if (cells <= 3072 * 3072) {
         *kernel = TWS_KERNEL_TILE_64x64;
         *k = 5;
     } else if (cells <= 4096 * 4096) {
