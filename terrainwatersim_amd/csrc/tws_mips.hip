@@ -67,6 +67,11 @@ constexpr int kMipReach = 40;  // what it computes of that level, at most: a las
                                // block owns 32 + 7, an odd side needs 3 + 2 * 18
 constexpr int kMipRows = 8;    // wavefronts of a work group, a row of texels each
 
+struct MipAxis {
+    int i0, i1;
+    float t;
+};
+
 struct MipSpan {
     int first, own, end;  // computed: [first, end), written: [first, own)
 };
@@ -95,6 +100,9 @@ __global__ void __launch_bounds__(kWave * kMipRows)
 k_mip_block(GridDesc g, int parity, float gb, const float4* __restrict__ src, int ws, int hs,
             float4* __restrict__ dst, int levels) {
     __shared__ float2 s_mip[2][kMipReach * kMipReach];  // {r, a}
+    // sample positions of a block's columns and rows, every level: worked out
+    // once, since a position between texels takes a division in FP64
+    __shared__ MipAxis s_axis[2][kMipLevels][kMipReach];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int side = kMipSide >> (levels - 1);
     const bool last_x = blockIdx.x + 1 == gridDim.x, last_y = blockIdx.y + 1 == gridDim.y;
@@ -120,15 +128,29 @@ k_mip_block(GridDesc g, int parity, float gb, const float4* __restrict__ src, in
     for (int l = 0; l < kMipLevels; ++l) {
         if (l >= levels) break;
         const int sw = l == 0 ? ws : w[l > 0 ? l - 1 : 0], sh = l == 0 ? hs : h[l > 0 ? l - 1 : 0];
+        if (wave == 2 * l && sx[l].first + lane < sx[l].end) {
+            MipAxis& x = s_axis[0][l][lane];
+            mip_axis(sx[l].first + lane, sw, w[l], x.i0, x.i1, x.t);
+        }
+        if (wave == 2 * l + 1 && sy[l].first + lane < sy[l].end) {
+            MipAxis& y = s_axis[1][l][lane];
+            mip_axis(sy[l].first + lane, sh, h[l], y.i0, y.i1, y.t);
+        }
+    }
+    static_assert(kMipRows >= 2 * kMipLevels, "a wavefront for each axis of each level");
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < kMipLevels; ++l) {
+        if (l >= levels) break;
         const int i = sx[l].first + lane;
         if (i < sx[l].end) {
-            int x0, x1;
-            float tx;
-            mip_axis(i, sw, w[l], x0, x1, tx);
+            const MipAxis ax = s_axis[0][l][lane];
+            const int x0 = ax.i0, x1 = ax.i1;
+            const float tx = ax.t;
             for (int j = sy[l].first + wave; j < sy[l].end; j += kMipRows) {
-                int y0, y1;
-                float ty;
-                mip_axis(j, sh, h[l], y0, y1, ty);
+                const MipAxis ay = s_axis[1][l][j - sy[l].first];
+                const int y0 = ay.i0, y1 = ay.i1;
+                const float ty = ay.t;
                 float2 v;
                 if (l == 0 && PLANES) {
                     const int64_t r0 = (int64_t)y0 * g.pitch, r1 = (int64_t)y1 * g.pitch;
@@ -228,7 +250,15 @@ int grid_mips(GridState& g, float gb_fill, float* dst, size_t capacity_floats, h
             hipLaunchKernelGGL(k_mip_tail, dim3(1), dim3(kTailThreads), 0, s, prev, ws, hs, out);
             left = 0;
         } else {
-            const int n = left < kMipLevels ? left : kMipLevels, side = kMipSide >> (n - 1);
+            // Four levels where that leaves no more than the tail takes, else three:
+            // as many launches up to 8192^2, and a block of an odd side computes
+            // 35 x 35 texels of its first level instead of 39 x 39.  us a chain at
+            // 4059 x 5027, with four levels and with three: 82.0 and
+            // 77.6 (a launch per level: 76.0); 4096^2 58.5 -> 47.6 against that, 1024^2
+            // 17.5 -> 10.9, 256^2 10.4 -> 9.1.
+            int n = left < kMipLevels ? left : kMipLevels;
+            if (n == kMipLevels && (int64_t)(ws >> n) * (hs >> n) > kTailTexels) n = kMipLevels - 1;
+            const int side = kMipSide >> (n - 1);
             const int wl = ws >> n > 0 ? ws >> n : 1, hl = hs >> n > 0 ? hs >> n : 1;
             const dim3 grid((wl + side - 1) / side, (hl + side - 1) / side);
             if (prev)
