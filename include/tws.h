@@ -67,9 +67,8 @@ extern "C" {
                                    directed flow (0); the brush and the rain
                                    reach only columns < 32*(W/32) and rows
                                    < 32*(H/32).  Where W and H are multiples of
-                                   32 this is ZERO.  Other sizes step on the
-                                   two-pass kernels, single grids only (a batch
-                                   refuses them). */
+                                   32 this is ZERO.  Other sizes are single
+                                   grids only (a batch refuses them). */
 
 /* Per-step constants of the SimulationParameters block
  * (simulationCommon.glsl:1-13) plus the boundary mode.  F, K and C must be

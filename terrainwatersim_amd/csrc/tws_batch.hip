@@ -33,6 +33,7 @@
 #include "tws_grid.hpp"
 #include "tws_pool.hpp"
 #include "tws_runtime.hpp"
+#include "tws_transfer.hpp"
 
 using namespace tws;
 
@@ -108,6 +109,7 @@ struct CapPlan {
 }  // namespace
 
 struct tws_batch {
+    TransferUser transfers;
     hipStream_t stream = nullptr;
     bool own_stream = false;
     DevicePool pool;

@@ -7,6 +7,7 @@
 #include "tws_fbm.hpp"
 #include "tws_grid.hpp"
 #include "tws_runtime.hpp"
+#include "tws_transfer.hpp"
 
 namespace tws {
 
@@ -83,11 +84,16 @@ bool grid_tiles(int W, int H, int kernel, int k, int* tiles_x, int* tiles_y) {
 // at ~2 GB/s against ~17 GB/s for 1D ones.  A plane whose rows are padded
 // goes through `st` (>= W*H floats of device scratch) and a 2D copy on the
 // device.
+// `pageable`: the host array is the caller's, and the call waits for the copy.
 static hipError_t plane_h2d(float* plane, int64_t pitch, const float* host, int W, int H,
-                            float* st, hipStream_t s) {
+                            float* st, hipStream_t s, bool pageable) {
     const size_t row = sizeof(float) * (size_t)W;
-    if (pitch == W) return hipMemcpyAsync(plane, host, row * H, hipMemcpyHostToDevice, s);
-    hipError_t e = hipMemcpyAsync(st, host, row * H, hipMemcpyHostToDevice, s);
+    auto copy = [&](float* to) {
+        return pageable ? copy_to_device(to, host, row * H, s)
+                        : hipMemcpyAsync(to, host, row * H, hipMemcpyHostToDevice, s);
+    };
+    if (pitch == W) return copy(plane);
+    hipError_t e = copy(st);
     if (e == hipSuccess)
         e = hipMemcpy2DAsync(plane, sizeof(float) * (size_t)pitch, st, row, row, H,
                              hipMemcpyDeviceToDevice, s);
@@ -95,12 +101,16 @@ static hipError_t plane_h2d(float* plane, int64_t pitch, const float* host, int 
 }
 
 static hipError_t plane_d2h(float* host, const float* plane, int64_t pitch, int W, int H,
-                            float* st, hipStream_t s) {
+                            float* st, hipStream_t s, bool pageable) {
     const size_t row = sizeof(float) * (size_t)W;
-    if (pitch == W) return hipMemcpyAsync(host, plane, row * H, hipMemcpyDeviceToHost, s);
+    auto copy = [&](const float* from) {
+        return pageable ? copy_to_host(host, from, row * H, s)
+                        : hipMemcpyAsync(host, from, row * H, hipMemcpyDeviceToHost, s);
+    };
+    if (pitch == W) return copy(plane);
     hipError_t e = hipMemcpy2DAsync(st, row, plane, sizeof(float) * (size_t)pitch, row, H,
                                     hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(host, st, row * H, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = copy(st);
     return e;
 }
 
@@ -114,13 +124,12 @@ int grid_upload(GridState& g, const float* terrain, const float* depth, const fl
                 hipStream_t s) {
     float* st = g.staging();
     if (terrain)
-        TWS_HIP(plane_h2d(g.b, g.pitch, terrain, g.W, g.H, st, s), "upload: terrain");
+        TWS_HIP(plane_h2d(g.b, g.pitch, terrain, g.W, g.H, st, s, true), "upload: terrain");
     if (depth)
-        TWS_HIP(plane_h2d(g.d[g.parity], g.pitch, depth, g.W, g.H, st, s), "upload: depth");
+        TWS_HIP(plane_h2d(g.d[g.parity], g.pitch, depth, g.W, g.H, st, s, true), "upload: depth");
     const GridDesc gd = g.desc();
     if (flux4) {
-        TWS_HIP(hipMemcpyAsync(st, flux4, sizeof(float) * 4 * (size_t)g.W * g.H,
-                               hipMemcpyHostToDevice, s), "upload: flux");
+        TWS_HIP(copy_to_device(st, flux4, sizeof(float) * 4 * (size_t)g.W * g.H, s), "upload: flux");
         TWS_HIP(launch_deinterleave(gd, g.parity, st, s), "upload: deinterleave");
     } else {
         TWS_HIP(launch_zero_fill(g.f[g.parity][0], 4 * g.pitch * (int64_t)g.H, s),
@@ -135,16 +144,16 @@ int grid_upload_async(GridState& g, const float* terrain, const float* depth, hi
     // a grid being admitted is not stepping: its idle flux set is free scratch
     float* st = g.staging();
     if (terrain)
-        TWS_HIP(plane_h2d(g.b, g.pitch, terrain, g.W, g.H, st, s), "upload: terrain");
+        TWS_HIP(plane_h2d(g.b, g.pitch, terrain, g.W, g.H, st, s, false), "upload: terrain");
     if (depth)
-        TWS_HIP(plane_h2d(g.d[g.parity], g.pitch, depth, g.W, g.H, st, s), "upload: depth");
+        TWS_HIP(plane_h2d(g.d[g.parity], g.pitch, depth, g.W, g.H, st, s, false), "upload: depth");
     TWS_HIP(launch_zero_fill(g.f[g.parity][0], 4 * g.pitch * (int64_t)g.H, s), "upload: flux");
     TWS_HIP(launch_check_finite(g.desc(), g.parity, s), "upload: finite check");
     return TWS_OK;
 }
 
 int grid_download_depth_async(GridState& g, float* depth, hipStream_t s) {
-    TWS_HIP(plane_d2h(depth, g.d[g.parity], g.pitch, g.W, g.H, g.staging(), s), "download: depth");
+    TWS_HIP(plane_d2h(depth, g.d[g.parity], g.pitch, g.W, g.H, g.staging(), s, false), "download: depth");
     return TWS_OK;
 }
 
@@ -152,19 +161,17 @@ int grid_download(GridState& g, float* depth, float* flux4, float* velocity2, hi
     const GridDesc gd = g.desc();
     float* st = g.staging();
     if (depth) {
-        TWS_HIP(plane_d2h(depth, g.d[g.parity], g.pitch, g.W, g.H, st, s), "download: depth");
+        TWS_HIP(plane_d2h(depth, g.d[g.parity], g.pitch, g.W, g.H, st, s, true), "download: depth");
         TWS_HIP(hipStreamSynchronize(s), "download: sync");  // st is reused below
     }
     if (flux4) {
         TWS_HIP(launch_interleave(gd, g.parity, st, s), "download: interleave");
-        TWS_HIP(hipMemcpyAsync(flux4, st, sizeof(float) * 4 * (size_t)g.W * g.H,
-                               hipMemcpyDeviceToHost, s), "download: flux");
+        TWS_HIP(copy_to_host(flux4, st, sizeof(float) * 4 * (size_t)g.W * g.H, s), "download: flux");
         TWS_HIP(hipStreamSynchronize(s), "download: sync");
     }
     if (velocity2) {
         TWS_HIP(launch_velocity(gd, g.parity, st, s), "download: velocity");
-        TWS_HIP(hipMemcpyAsync(velocity2, st, sizeof(float) * 2 * (size_t)g.W * g.H,
-                               hipMemcpyDeviceToHost, s), "download: velocity copy");
+        TWS_HIP(copy_to_host(velocity2, st, sizeof(float) * 2 * (size_t)g.W * g.H, s), "download: velocity copy");
     }
     TWS_HIP(hipStreamSynchronize(s), "download: sync");
     return TWS_OK;
@@ -176,13 +183,13 @@ int grid_upload_reference(GridState& g, const float* terrain_rgba, const float* 
     float* st = g.staging();
     const size_t bytes = sizeof(float) * 4 * (size_t)g.W * g.H;
     if (terrain_rgba) {
-        TWS_HIP(hipMemcpyAsync(st, terrain_rgba, bytes, hipMemcpyHostToDevice, s),
+        TWS_HIP(copy_to_device(st, terrain_rgba, bytes, s),
                 "upload_reference: terrain");
         TWS_HIP(launch_ref_unpack(gd, g.parity, st, nullptr, g.b, s),
                 "upload_reference: unpack terrain");
     }
     if (flow_rgba) {
-        TWS_HIP(hipMemcpyAsync(st, flow_rgba, bytes, hipMemcpyHostToDevice, s),
+        TWS_HIP(copy_to_device(st, flow_rgba, bytes, s),
                 "upload_reference: flow");
         TWS_HIP(launch_ref_unpack(gd, g.parity, nullptr, st, g.b, s),
                 "upload_reference: unpack flow");
@@ -200,23 +207,20 @@ int grid_download_reference(GridState& g, float* terrain_rgba, float gb_fill, fl
     if (terrain_rgba) {
         TWS_HIP(launch_ref_pack(gd, g.parity, gb_fill, st, nullptr, nullptr, s),
                 "download_reference: pack terrain");
-        TWS_HIP(hipMemcpyAsync(terrain_rgba, st, sizeof(float) * 4 * cells,
-                               hipMemcpyDeviceToHost, s), "download_reference: terrain");
+        TWS_HIP(copy_to_host(terrain_rgba, st, sizeof(float) * 4 * cells, s), "download_reference: terrain");
         TWS_HIP(hipStreamSynchronize(s), "download_reference: sync");
     }
     if (flow_rgba) {
         TWS_HIP(launch_ref_pack(gd, g.parity, gb_fill, nullptr, st, nullptr, s),
                 "download_reference: pack flow");
-        TWS_HIP(hipMemcpyAsync(flow_rgba, st, sizeof(float) * 4 * cells, hipMemcpyDeviceToHost,
-                               s), "download_reference: flow");
+        TWS_HIP(copy_to_host(flow_rgba, st, sizeof(float) * 4 * cells, s), "download_reference: flow");
         TWS_HIP(hipStreamSynchronize(s), "download_reference: sync");
     }
     if (flowmap) {
         uint16_t* st16 = reinterpret_cast<uint16_t*>(st);
         TWS_HIP(launch_ref_pack(gd, g.parity, gb_fill, nullptr, nullptr, st16, s),
                 "download_reference: pack flowmap");
-        TWS_HIP(hipMemcpyAsync(flowmap, st16, sizeof(uint16_t) * 2 * cells,
-                               hipMemcpyDeviceToHost, s), "download_reference: flowmap");
+        TWS_HIP(copy_to_host(flowmap, st16, sizeof(uint16_t) * 2 * cells, s), "download_reference: flowmap");
     }
     TWS_HIP(hipStreamSynchronize(s), "download_reference: sync");
     return TWS_OK;

@@ -14,10 +14,9 @@
 // between texels 2i and 2i+1 and matches llvmpipe bit for bit; other ratios
 // use the exact sample position (double, t rounded once to float).
 //
-// Level 1 reads the b and d planes of the current state (8 B per level-0
-// cell) and writes 16 B per level-1 texel; level l > 1 reads level l-1.  A
-// wave covers 64 consecutive texels of one row, so the source rows are read
-// as contiguous 512-byte runs.
+// Blocks of three or four levels are made from one read of the planes, or of the
+// last level made, in LDS (k_mip_block); the small end of the chain is one work
+// group's (k_mip_tail).
 
 #include <hip/hip_runtime.h>
 
@@ -186,7 +185,7 @@ k_mip_block(GridDesc g, int parity, float gb, const float4* __restrict__ src, in
 // The small end of the chain in one work group: every level from one of at
 // most kTailTexels texels down to 1x1, level after level, each read back
 // from the chain buffer that this work group wrote before the barrier.  The
-// per-texel arithmetic is k_mip_next's; the levels cost one launch instead of
+// per-texel arithmetic is the blocks'; the levels cost one launch instead of
 // one each (they are bound by launch latency, not by bytes).
 constexpr int kTailThreads = 1024;
 constexpr int kTailTexels = 64 * 64;

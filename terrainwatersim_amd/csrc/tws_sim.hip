@@ -11,10 +11,12 @@
 #include "tws.h"
 #include "tws_grid.hpp"
 #include "tws_runtime.hpp"
+#include "tws_transfer.hpp"
 
 using namespace tws;
 
 struct tws_sim {
+    TransferUser transfers;
     GridState g;
     hipStream_t stream = nullptr;
     bool own_stream = false;
