@@ -26,8 +26,11 @@ namespace {
 // 4, 2, 1/2 4310; 4, 2, 1 3360; 8, 2, 1 3580; 4, 2, 2 3070; 4, 1, 4 2990; 4, 2, 4 2990.
 constexpr size_t kChunk = 4 << 20;
 constexpr int kThreads = 4;  // a slot each
-// Copies below this stay with the runtime: starting the threads costs more.
-constexpr size_t kStagedMin = 3 << 20;
+// Copies below this stay with the runtime: starting the threads and their few
+// large chunks costs more.  ms by MiB, runtime and threads: up 16 0.51, 0.55; 24
+// 0.76, 0.75; 32 1.15, 0.96; 128 4.9, 3.4; down 4 0.24, 0.27; 6 0.37, 0.31; 16 1.02,
+// 0.57; 32 3.6, 1.6; 128 13.2, 4.2.
+constexpr size_t kStagedUp = 24 << 20, kStagedDown = 5 << 20;
 constexpr int kMaxIdle = 2;  // stagings kept while no copy uses them
 
 struct Staging {
@@ -111,7 +114,7 @@ hipError_t copy(char* device, char* host, size_t bytes, hipStream_t s) {
         return UP ? hipMemcpyAsync(device, host, bytes, hipMemcpyHostToDevice, s)
                   : hipMemcpyAsync(host, device, bytes, hipMemcpyDeviceToHost, s);
     };
-    if (bytes < kStagedMin) return direct();
+    if (bytes < (UP ? kStagedUp : kStagedDown)) return direct();
     // memory that is pinned already needs no copy on the way
     hipPointerAttribute_t attr{};
     if (hipPointerGetAttributes(&attr, host) != hipSuccess) (void)hipGetLastError();

@@ -31,10 +31,11 @@ def there_and_back(gpu, W, H, seed, wrap=lambda a: a):
         assert np.array_equal(out["depth"], d[::-1]) and np.array_equal(out["flux"], f[::-1])
 
 
-# flux, and planes with rows of 1024 floats, of 3 MiB less a row, 3 MiB, a row
-# more, 8 whole chunks, and sides that divide nothing
-@pytest.mark.parametrize("W,H", [(1024, 191), (1024, 192), (1024, 193), (1024, 767), (1024, 768),
-                                 (1024, 2048), (1331, 1024), (997, 1403)])
+# flux and planes a row less than 5 MiB (downloads) and 24 MiB (uploads), as much
+# and a row more, whole chunks, and sides that divide nothing
+@pytest.mark.parametrize("W,H", [(1024, 319), (1024, 320), (1024, 321), (1024, 1280), (1024, 1535),
+                                 (1024, 1536), (1024, 1537), (1024, 2048), (1331, 1024),
+                                 (1403, 1397)])
 def test_large_copies_are_exact(gpu, W, H):
     there_and_back(gpu, W, H, W + H)
 
@@ -44,7 +45,7 @@ def test_copies_from_several_threads(gpu):
 
     def work(i):
         try:
-            there_and_back(gpu, 900 + 13 * i, 700 + 7 * i, i)
+            there_and_back(gpu, 1300 + 13 * i, 1300 + 7 * i, i)
         except BaseException as e:  # noqa: BLE001
             failed.append(e)
 
@@ -69,7 +70,7 @@ def test_pinned_arrays(gpu):
         return out
 
     try:
-        there_and_back(gpu, 1024, 800, 5, pinned)
+        there_and_back(gpu, 1024, 1600, 5, pinned)
     finally:
         for p in kept:
             hip.hipHostFree(p)
