@@ -154,6 +154,9 @@ int step_grid(GridState& gs, int kernel, int k, int32_t n, hipStream_t stream, h
             return fail(TWS_ERR_INVALID, "step: bad launch config %d/%d", kernel, kk);
         g.tile_begin = 0;
         g.steps = levels;
+        // one group of columns is the row-major order, with a division less
+        // (256^2 rain, 1000 steps, 1568 -> 1545 us)
+        if (g.tile_group >= g.tiles_x) g.tile_group = 0;
         const int64_t tiles = (int64_t)g.tiles_x * g.tiles_y;
         DryMaps dry;
         if (kk == k && levels == k && full > 2 && tile_looks(kernel, k) && tiles >= kDryTiles &&
