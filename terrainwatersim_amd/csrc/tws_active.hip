@@ -39,8 +39,9 @@ constexpr int kPlanWords = 6144;      // words k_plan can plan (in LDS)
 constexpr int kReachBands = kActiveReach / kBand;
 // Rounds (a survey and its plan) until a state found all wet is looked at
 // again.  MI355X, 100 steps of the wet 4096^2 sheet (3.9 ms, 4 rounds of k = 6):
-// 2.0% for the rounds when each looks, 1.0% when only the first does.
-constexpr int kFullRounds = 4;
+// 2.0% for the rounds when each looks, 1.0% when only the first does; 1000 steps
+// in one call 34.5 ms looking every 4 rounds, 34.3 every 8.
+constexpr int kFullRounds = 8;
 constexpr int kMinRows = 16;          // shortest segment worth a wavefront
 
 // Words of a grid's masks: any | left | right | active, strips x words each.
@@ -288,11 +289,18 @@ k_plan(GridDesc g1, const GridDesc* __restrict__ grids, const int* __restrict__ 
     // times where a segment would run past max_rows.
     const int rounds = max(1, (s_rows / slots + max_rows - 1) / max_rows);
     const int free_slots = slots * rounds - s_runs;
-    if (words > kPlanWords || free_slots <= 0 || s_rows >= s_all - s_all / 8) {
+    // Only where a wavefront sweeps an eighth less than in the static plan, the 4 k
+    // rows of a segment's ramps counted: fragments of active rows take slots and
+    // ramps of their own, and surveying them takes some 5% of the launches.
+    // (4096^2 sheet with a tenth of it dry, 1000 steps: 35.3 ms listed, 33.3 static.)
+    const int all_rounds = max(1, (s_all / slots + max_rows - 1) / max_rows);
+    const int all_len = (s_all + slots * all_rounds - 1) / (slots * all_rounds);
+    const int len = free_slots > 0 ? max(kMinRows, (s_rows + free_slots - 1) / free_slots) : 0;
+    if (words > kPlanWords || free_slots <= 0 ||
+        (int64_t)(len + 4 * k) * rounds * 8 > (int64_t)(all_len + 4 * k) * all_rounds * 7) {
         if (tid == 0) *count = -1;
         return;
     }
-    const int len = max(kMinRows, (s_rows + free_slots - 1) / free_slots);
     // Calls run(first band, rows) for the runs of a word's bands; `below`: rows
     // of the grid from the word's first on.
     auto each_run = [](uint64_t m, int below, auto run) {
